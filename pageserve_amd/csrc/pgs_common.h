@@ -64,6 +64,33 @@ __device__ __forceinline__ uint32_t pack_bf16x2(float a, float b) {
   return __builtin_bit_cast(uint32_t, v);
 }
 
+template <int OUT>  // PGS_DTYPE_*
+__device__ __forceinline__ void store_dequant(void* out, int64_t e, float v) {
+  if constexpr (OUT == PGS_DTYPE_F32)
+    reinterpret_cast<float*>(out)[e] = v;
+  else if constexpr (OUT == PGS_DTYPE_BF16)
+    reinterpret_cast<uint16_t*>(out)[e] = f32_to_bf16_bits(v);
+  else
+    reinterpret_cast<_Float16*>(out)[e] = static_cast<_Float16>(v);
+}
+
+// 16 bytes of output from element e on: four fp32 or eight 16-bit values
+template <int OUT>
+__device__ __forceinline__ void store_dequant16(void* out, int64_t e, const float* f) {
+  if constexpr (OUT == PGS_DTYPE_F32) {
+    *reinterpret_cast<f32x4*>(reinterpret_cast<float*>(out) + e) = f32x4{f[0], f[1], f[2], f[3]};
+  } else if constexpr (OUT == PGS_DTYPE_BF16) {
+    *reinterpret_cast<u32x4*>(reinterpret_cast<uint16_t*>(out) + e) =
+        u32x4{pack_bf16x2(f[0], f[1]), pack_bf16x2(f[2], f[3]), pack_bf16x2(f[4], f[5]), pack_bf16x2(f[6], f[7])};
+  } else {
+    typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
+    f16x8 v;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) v[i] = static_cast<_Float16>(f[i]);
+    *reinterpret_cast<f16x8*>(reinterpret_cast<_Float16*>(out) + e) = v;
+  }
+}
+
 // x * sigmoid(x) in fp32 (F.silu): x / (1 + e^-x) with the hardware
 // base-2 exponential (v_exp_f32, e^-x = 2^(-x log2 e)) and the hardware
 // reciprocal (v_rcp_f32), each within about one fp32 ulp, in about 5

@@ -250,3 +250,48 @@ def test_non_finite_rows_follow_the_reference(gpu, dtype):
     qw = Q.QuantizedWeight(torch.from_numpy(w).to(gpu) if dtype == torch.float32 else
                            torch.from_numpy(O.f32_to_bf16_bits(w).view(np.int16).copy()).view(torch.bfloat16).to(gpu))
     np.testing.assert_array_equal(qw.q.cpu().numpy(), q_ref)
+
+
+@pytest.mark.parametrize("n,k", [(1, 4), (8, 8), (9, 1024), (16, 1032), (23, 2048), (7, 2056), (33, 5120), (15, 5128),
+                                 (17, 12288), (3, 12296), (40, 72)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_tile_kernel_edges(gpu, n, k, dtype):
+    """The smallest, full and just exceeded register tiles of the eight-row
+    quantizer and the remainders of its rows and columns: row-major and packed
+    bytes (padding included), with a zero, a NaN and an infinite row."""
+    w = random_matrix(6000 + n + k, n, k) if n >= 4 else weights(11, n, k)
+    if n >= 7:
+        w[2], w[4, k - 1], w[6, 0] = 0.0, np.nan, -np.inf
+    if dtype == torch.bfloat16:
+        w = O.round_to_bf16(w)
+    q_ref, s_ref = O.quantize_per_channel(w)
+    q, s = _gpu_quant(w, gpu, dtype)
+    np.testing.assert_array_equal(q, q_ref)
+    np.testing.assert_array_equal(s, s_ref)  # (NaN equal to NaN)
+    qw = Q.QuantizedWeight(torch.from_numpy(w).to(gpu).to(dtype))
+    np.testing.assert_array_equal(qw.qp.cpu().numpy(), O.pack_tiles(q_ref))
+    np.testing.assert_array_equal(qw.scale.cpu().numpy(), s_ref)
+
+
+@pytest.mark.parametrize("n,k", [(5, 3), (9, 4), (77, 5), (50, 7), (64, 8), (33, 9), (11, 12), (70, 1031), (16, 4104)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+def test_dequantize_pieces_across_rows(gpu, n, k, dtype):
+    """Output pieces that start in one row and end in the next, a last short
+    piece, and rows shorter than a piece; the packed form at the same shapes."""
+    q = np.random.default_rng(n * 31 + k).integers(-127, 128, (n, k)).astype(np.int8)
+    s = np.random.default_rng(k).uniform(1e-4, 1e-2, (n, 1)).astype(np.float32)
+    ref = torch.from_numpy(q.astype(np.float32) * s).to(dtype)
+    out = Q.dequantize(torch.from_numpy(q).to(gpu), torch.from_numpy(s).to(gpu), dtype)
+    assert torch.equal(out.cpu(), ref)
+    qw = Q.QuantizedWeight(torch.zeros((n, k), dtype=dtype, device=gpu))
+    qw.q, qw.scale = torch.from_numpy(q).to(gpu), torch.from_numpy(s).to(gpu)
+    assert torch.equal(qw.dense().cpu(), ref)
+
+
+def test_dequantize_above_32_bit_indices(gpu):
+    n, k = 65600, 65544
+    q = torch.randint(-127, 128, (64, k), dtype=torch.int8, device=gpu).repeat(n // 64, 1)
+    s = torch.rand((n, 1), device=gpu) * 0.01
+    out = Q.dequantize(q, s, torch.bfloat16)
+    for r in (slice(0, 40), slice(n // 2, n // 2 + 40), slice(n - 40, n)):
+        assert torch.equal(out[r], (q[r].float() * s[r]).to(torch.bfloat16))
