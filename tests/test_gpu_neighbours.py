@@ -23,7 +23,8 @@ from pageserve_amd import quantization as Q
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("m,k", [(1, 2048), (16, 2048), (512, 2048), (7, 896), (3, 100), (2, 11008), (1, 8)])
+@pytest.mark.parametrize("m,k", [(1, 2048), (16, 2048), (512, 2048), (7, 896), (3, 100), (2, 11008), (1, 8),
+                                 (3, 2056), (2, 4096), (5, 4104), (2, 8192), (3, 8200)])
 def test_rmsnorm_matches_oracle(gpu, m, k):
     rng = np.random.default_rng(m * 100 + k)
     x = O.round_to_bf16(rng.standard_normal((m, k), dtype=np.float32) * np.float32(2.0))
