@@ -268,9 +268,9 @@ int pgs_w8a16_swiglu(const void* x, const int8_t* qp_gate, const float* s_gate,
 /*
  * Replaces h = rms_norm(x, weight, eps) followed by the q/k/v projections of
  * h -- engine/model.py:166 (rms_norm at :29-34) and :168-170 -- with one
- * launch where the plan allows (m <= 4 tokens, K % 64 == 0, no K split, bf16
- * outputs, 16-byte aligned norm weight): the kernel normalises the
- * activations it stages, with the reference's roundings
+ * launch where the plan allows (m <= 32 tokens, K % 64 == 0 and at most 2048
+ * above 4 tokens, no K split, bf16 outputs, 16-byte aligned norm weight): the
+ * kernel normalises the activations it loads, with the reference's roundings
  * (h = bf16(weight * bf16(x * r)), r = 1/sqrt(mean(x^2) + eps) in fp32);
  * otherwise pgs_rmsnorm into the workspace, then pgs_w8a16_linear_group.
  * The fp32 sum of squares is formed in a fixed order (deterministic) that
@@ -293,6 +293,21 @@ int pgs_w8a16_rmsnorm_swiglu(const void* x, const void* norm_weight, float eps,
                              const int8_t* qp_up, const float* s_up, void* act,
                              int64_t m, int64_t n, int64_t k, void* workspace,
                              size_t workspace_bytes, void* stream);
+
+/*
+ * pgs_w8a16_rmsnorm_linear_group for q, k and v (outs[0..2], bf16 outputs),
+ * then RoPE of q and k (engine/model.py:166-173): the outputs are
+ * apply_rope(q), apply_rope(k) and v, with the reference's roundings (the bf16
+ * projection, then pgs_rope's three).  cos / sin: bf16 [m, head_dim]; outs[0].n
+ * and outs[1].n are whole heads of head_dim.  One launch at up to 32 tokens
+ * where the norm runs inside the projection and head_dim % 32 == 0 (the two
+ * halves of a head are then computed side by side); the separate kernels
+ * otherwise.  Workspace: pgs_w8a16_rmsnorm_workspace_bytes of the three.
+ */
+int pgs_w8a16_rmsnorm_qkv_rope(const void* x, const void* norm_weight, float eps,
+                               const pgs_linear_out* outs, const void* cos,
+                               const void* sin, int64_t head_dim, int64_t m, int64_t k,
+                               void* workspace, size_t workspace_bytes, void* stream);
 
 /*
  * Workspace bytes a linear call needs (0 = none): n[0..n_outs-1] are the

@@ -99,6 +99,8 @@ SIGNATURES = {
     "pgs_w8a16_workspace_bytes": (_SZ, [_I64, ctypes.POINTER(_I64), _INT, _I64, _INT]),
     "pgs_w8a16_rmsnorm_linear_group": (_INT, [_VP, _VP, ctypes.c_float, ctypes.POINTER(LinearOut), _INT, _INT,
                                               _I64, _I64, _VP, _SZ, _VP]),
+    "pgs_w8a16_rmsnorm_qkv_rope": (_INT, [_VP, _VP, ctypes.c_float, ctypes.POINTER(LinearOut), _VP, _VP, _I64, _I64,
+                                          _I64, _VP, _SZ, _VP]),
     "pgs_w8a16_rmsnorm_swiglu": (_INT, [_VP, _VP, ctypes.c_float, _VP, _VP, _VP, _VP, _VP, _I64, _I64, _I64, _VP,
                                         _SZ, _VP]),
     "pgs_w8a16_rmsnorm_workspace_bytes": (_SZ, [_I64, ctypes.POINTER(_I64), _INT, _I64, _INT]),

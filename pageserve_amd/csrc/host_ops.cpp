@@ -82,12 +82,20 @@ at::Tensor check_norm(const Opt& w, int64_t k, const at::Device& dev, const char
   return aligned(t.reshape({k}), 16);
 }
 
+// RoPE of a q|k|v call's first two outputs: cos / sin bf16 [m, head_dim].
+struct Rope {
+  at::Tensor cos, sin;
+  int64_t head_dim = 0;
+};
+
 // One or more projections of the same input (linear, linear_group, and with
-// a single member the residual / out forms; norm_w: rms_norm fused in front).
-std::vector<at::Tensor> linear(const at::Tensor& x, const std::vector<at::Tensor>& qps,
-                               const std::vector<at::Tensor>& scales, const std::vector<Opt>& biases,
-                               const std::vector<int64_t>& ns, int64_t k, bool out_f32, const Opt& residual,
-                               const Opt& out, const Opt& norm_w, double eps, int64_t ws_ptr, int64_t ws_bytes) {
+// a single member the residual / out forms; norm_w: rms_norm fused in front;
+// rope: with norm_w and three members, RoPE behind the first two).
+std::vector<at::Tensor> linear_impl(const at::Tensor& x, const std::vector<at::Tensor>& qps,
+                                    const std::vector<at::Tensor>& scales, const std::vector<Opt>& biases,
+                                    const std::vector<int64_t>& ns, int64_t k, bool out_f32, const Opt& residual,
+                                    const Opt& out, const Opt& norm_w, double eps, int64_t ws_ptr, int64_t ws_bytes,
+                                    const Rope* rope) {
   const size_t g = qps.size();
   if (g < 1 || g > PGS_MAX_GROUP || scales.size() != g || biases.size() != g || ns.size() != g)
     value_error("linear_group takes 1.." + std::to_string(PGS_MAX_GROUP) + " weights");
@@ -148,7 +156,10 @@ std::vector<at::Tensor> linear(const at::Tensor& x, const std::vector<at::Tensor
   void* ws = reinterpret_cast<void*>(static_cast<uintptr_t>(ws_ptr));
   const int ydt = out_f32 ? PGS_DTYPE_F32 : PGS_DTYPE_BF16;
   int rc;
-  if (nw.defined())
+  if (rope)
+    rc = pgs_w8a16_rmsnorm_qkv_rope(ptr(x2), nw.data_ptr(), static_cast<float>(eps), outs, ptr(rope->cos),
+                                    ptr(rope->sin), rope->head_dim, m, k, ws, static_cast<size_t>(ws_bytes), st);
+  else if (nw.defined())
     rc = pgs_w8a16_rmsnorm_linear_group(ptr(x2), nw.data_ptr(), static_cast<float>(eps), outs, static_cast<int>(g), ydt,
                                         m, k, ws, static_cast<size_t>(ws_bytes), st);
   else if (res.defined() || out.has_value())
@@ -160,6 +171,26 @@ std::vector<at::Tensor> linear(const at::Tensor& x, const std::vector<at::Tensor
   if (x.dim() != 2)
     for (size_t i = 0; i < g; ++i) ys[i] = ys[i].view(out_shape(x, ns[i]));
   return ys;
+}
+
+std::vector<at::Tensor> linear(const at::Tensor& x, const std::vector<at::Tensor>& qps,
+                               const std::vector<at::Tensor>& scales, const std::vector<Opt>& biases,
+                               const std::vector<int64_t>& ns, int64_t k, bool out_f32, const Opt& residual,
+                               const Opt& out, const Opt& norm_w, double eps, int64_t ws_ptr, int64_t ws_bytes) {
+  return linear_impl(x, qps, scales, biases, ns, k, out_f32, residual, out, norm_w, eps, ws_ptr, ws_bytes, nullptr);
+}
+
+// rms_norm, q|k|v and RoPE of q and k (one launch where the plan allows).
+// cos / sin: bf16 [m, head_dim] on the weights' device (checked by the caller).
+std::vector<at::Tensor> qkv_rope(const at::Tensor& x, const std::vector<at::Tensor>& qps,
+                                 const std::vector<at::Tensor>& scales, const std::vector<Opt>& biases,
+                                 const std::vector<int64_t>& ns, int64_t k, const at::Tensor& norm_w, double eps,
+                                 const at::Tensor& cos, const at::Tensor& sin, int64_t head_dim, int64_t ws_ptr,
+                                 int64_t ws_bytes) {
+  if (qps.size() != 3) value_error("qkv_rope takes the q, k and v weights");
+  const Rope rope{aligned(cos, 2), aligned(sin, 2), head_dim};
+  return linear_impl(x, qps, scales, biases, ns, k, false, c10::nullopt, c10::nullopt, norm_w, eps, ws_ptr, ws_bytes,
+                     &rope);
 }
 
 // One projection (linear and its residual / out forms): the group path
@@ -203,5 +234,6 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, mod) {
   mod.def("abi_version", &pgs_abi_version);
   mod.def("linear", &linear, "one or more W8A16 projections of the same input");
   mod.def("linear1", &linear1, "one W8A16 projection");
+  mod.def("qkv_rope", &qkv_rope, "rms_norm, q|k|v projections and RoPE of q and k");
   mod.def("swiglu", &swiglu, "fused gate/up/silu*up");
 }

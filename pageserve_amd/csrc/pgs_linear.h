@@ -35,6 +35,11 @@ struct Problem {
   unsigned long long* pairs;  // zeroed pair slots (skinny two-way split), or null
   const uint16_t* norm_w;     // rms_norm weight fused in front of the linear (bf16 [k]), or null
   float eps;
+  // RoPE of members 0 and 1 (q and k of a q|k|v group) in the epilogue: cos /
+  // sin bf16 [m, rope_hd], or null
+  const uint16_t* rope_cos;
+  const uint16_t* rope_sin;
+  int rope_hd;
   // Row-argmax mode (fp32 single matrix, skinny kernel, no K split): instead
   // of the outputs, workgroup b writes the key of its best output of token t
   // to keys[b * m + t] (argmax_key); null otherwise
@@ -75,8 +80,12 @@ SkinnyPlan plan_skinny(int m, int k, int nmat, int tiles, bool can_split);
 int64_t skinny_grid(const SkinnyPlan& p);
 size_t skinny_partial_bytes(const SkinnyPlan& p, int nmat);
 // whether the skinny kernel can apply rms_norm to its staged activations
-// (bf16 output, m <= 4, K % 64 == 0, no K split, an issue-once shape)
+// (bf16 output, K % 64 == 0, no K split, an issue-once shape whose registers
+// and LDS hold it)
 bool skinny_norm_fusable(const SkinnyPlan& p, int m, int k, bool out_f32, int nmat);
+// whether a launch with the fused norm can also rotate its first two members
+// (unfolded tiles; whole heads of a multiple of 32 dimensions)
+bool skinny_rope_fusable(const SkinnyPlan& p, int hd, const GroupArgs& a);
 int launch_skinny(Problem& p, const SkinnyPlan& plan, hipStream_t st);
 
 // pgs_w8a16_linear_group with the entry point's name `fn` in its messages

@@ -54,24 +54,8 @@ size_t norm_offset(size_t linear_bytes) {
   return (std::max(linear_bytes, kPairBytes) + 255) & ~static_cast<size_t>(255);
 }
 
-int run(Problem& p, void* workspace, size_t ws_bytes, hipStream_t st) {
-  if (int rc = require_device("w8a16 linear", st)) return rc;
+int run_plan(Problem& p, const Plan& plan, size_t need, void* workspace, size_t ws_bytes, hipStream_t st) {
   const int members = (p.nmat == 2) ? 1 : p.args.n_outs;
-  const Plan plan = make_plan(p.m, p.k, p.nmat, p.args.n, members, workspace != nullptr);
-  const size_t need = workspace_bytes(plan, p.nmat);
-  if (p.norm_w && !(plan.skinny && skinny_norm_fusable(plan.sk, p.m, p.k, p.out_f32, p.nmat) && aligned(p.norm_w, 16))) {
-    // rms_norm as its own kernel into the workspace, then the plain linear
-    const size_t off = norm_offset(need), bytes = static_cast<size_t>(p.m) * p.k * 2;
-    if (!workspace || ws_bytes < off + bytes)
-      return fail(PGS_ERR_INVALID_ARGUMENT, "w8a16 (rms_norm fused): workspace of %zu bytes, %zu needed", ws_bytes,
-                  off + bytes);
-    void* h = static_cast<char*>(workspace) + off;
-    int rc = pgs_rmsnorm(p.x, p.norm_w, p.eps, h, p.m, p.k, st);
-    if (rc) return rc;
-    p.x = static_cast<const uint16_t*>(h);
-    p.norm_w = nullptr;
-    ws_bytes = off;
-  }
   if (need > ws_bytes)
     return fail(PGS_ERR_INVALID_ARGUMENT, "w8a16: workspace of %zu bytes is smaller than the %zu this call needs",
                 ws_bytes, need);
@@ -91,6 +75,35 @@ int run(Problem& p, void* workspace, size_t ws_bytes, hipStream_t st) {
     return launch_skinny(p, plan.sk, st);
   }
   return launch_gemm(p, plan.gm, st);
+}
+
+int run(Problem& p, void* workspace, size_t ws_bytes, hipStream_t st) {
+  if (int rc = require_device("w8a16 linear", st)) return rc;
+  const int members = (p.nmat == 2) ? 1 : p.args.n_outs;
+  const Plan plan = make_plan(p.m, p.k, p.nmat, p.args.n, members, workspace != nullptr);
+  const size_t need = workspace_bytes(plan, p.nmat);
+  if (p.norm_w && !(plan.skinny && skinny_norm_fusable(plan.sk, p.m, p.k, p.out_f32, p.nmat) && aligned(p.norm_w, 16))) {
+    // rms_norm as its own kernel into the workspace, then the plain linear
+    const size_t off = norm_offset(need), bytes = static_cast<size_t>(p.m) * p.k * 2;
+    if (!workspace || ws_bytes < off + bytes)
+      return fail(PGS_ERR_INVALID_ARGUMENT, "w8a16 (rms_norm fused): workspace of %zu bytes, %zu needed", ws_bytes,
+                  off + bytes);
+    void* h = static_cast<char*>(workspace) + off;
+    int rc = pgs_rmsnorm(p.x, p.norm_w, p.eps, h, p.m, p.k, st);
+    if (rc) return rc;
+    p.x = static_cast<const uint16_t*>(h);
+    p.norm_w = nullptr;
+    ws_bytes = off;
+  }
+  if (p.rope_cos && !(p.norm_w && skinny_rope_fusable(plan.sk, p.rope_hd, p.args))) {
+    // RoPE as its own kernel, in place on the projections' outputs
+    Problem lin = p;
+    lin.rope_cos = lin.rope_sin = nullptr;
+    if (int rc = run_plan(lin, plan, need, workspace, ws_bytes, st)) return rc;
+    return pgs_rope(p.args.y[0], p.args.y[0], p.args.n[0] / p.rope_hd, p.args.y[1], p.args.y[1],
+                    p.args.n[1] / p.rope_hd, p.rope_cos, p.rope_sin, p.m, p.rope_hd, st);
+  }
+  return run_plan(p, plan, need, workspace, ws_bytes, st);
 }
 
 int check_common(const char* fn, const void* x, int64_t m, int64_t k) {
@@ -156,7 +169,8 @@ int check_norm(const char* fn, const void* w, float eps, int64_t m, int64_t k) {
 
 int linear_group_impl(const char* fn, const void* x, const pgs_linear_out* outs, const void* const* res, int n_outs,
                       int y_dtype, int64_t m, int64_t k, void* workspace, size_t workspace_bytes_, void* stream,
-                      const void* norm_w = nullptr, float eps = 0.f) {
+                      const void* norm_w = nullptr, float eps = 0.f, const void* cos = nullptr,
+                      const void* sin = nullptr, int64_t head_dim = 0) {
   int rc = check_common(fn, x, m, k);
   if (rc) return rc;
   if (!outs || n_outs < 1 || n_outs > PGS_MAX_GROUP)
@@ -171,6 +185,9 @@ int linear_group_impl(const char* fn, const void* x, const pgs_linear_out* outs,
   p.out_f32 = (y_dtype == PGS_DTYPE_F32);
   p.norm_w = static_cast<const uint16_t*>(norm_w);
   p.eps = eps;
+  p.rope_cos = static_cast<const uint16_t*>(cos);
+  p.rope_sin = static_cast<const uint16_t*>(sin);
+  p.rope_hd = static_cast<int>(head_dim);
   int used = 0;
   for (int i = 0; i < n_outs; ++i) {
     rc = check_member(fn, outs[i].qp, outs[i].scale, outs[i].bias, outs[i].y, outs[i].n, m, k);
@@ -286,6 +303,26 @@ extern "C" int pgs_w8a16_rmsnorm_linear_group(const void* x, const void* norm_we
   if (rc) return rc;
   return linear_group_impl(fn, x, outs, nullptr, n_outs, y_dtype, m, k, workspace, workspace_bytes_, stream,
                            norm_weight, eps);
+}
+
+extern "C" int pgs_w8a16_rmsnorm_qkv_rope(const void* x, const void* norm_weight, float eps,
+                                          const pgs_linear_out* outs, const void* cos, const void* sin,
+                                          int64_t head_dim, int64_t m, int64_t k, void* workspace,
+                                          size_t workspace_bytes_, void* stream) {
+  const char* fn = "pgs_w8a16_rmsnorm_qkv_rope";
+  int rc = check_norm(fn, norm_weight, eps, m, k);
+  if (rc) return rc;
+  if (!outs) return fail(PGS_ERR_INVALID_ARGUMENT, "%s: null pointer", fn);
+  if (head_dim < 2 || head_dim % 2 != 0 || head_dim > 0x10000)
+    return fail(PGS_ERR_INVALID_ARGUMENT, "%s: head_dim=%lld must be even and in [2, 65536]", fn, (long long)head_dim);
+  for (int i = 0; i < 3; ++i)
+    if (outs[i].n < 1 || (i < 2 && outs[i].n % head_dim != 0))
+      return fail(PGS_ERR_INVALID_ARGUMENT, "%s: output %d has n=%lld rows (whole heads of %lld wanted)", fn, i,
+                  (long long)outs[i].n, (long long)head_dim);
+  if (m > 0 && (!cos || !sin)) return fail(PGS_ERR_INVALID_ARGUMENT, "%s: null cos / sin", fn);
+  if (!aligned(cos, 2) || !aligned(sin, 2)) return fail(PGS_ERR_MISALIGNED, "%s: cos / sin misaligned", fn);
+  return linear_group_impl(fn, x, outs, nullptr, 3, PGS_DTYPE_BF16, m, k, workspace, workspace_bytes_, stream,
+                           norm_weight, eps, cos, sin, head_dim);
 }
 
 extern "C" int pgs_w8a16_rmsnorm_swiglu(const void* x, const void* norm_weight, float eps, const int8_t* q_gate,

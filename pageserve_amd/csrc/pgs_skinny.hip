@@ -104,6 +104,47 @@ constexpr int skinny_lds_bytes(int nw, int u, int nb, int nmat, int s, int xm, b
   return (xm > 0 ? nw * (xm >= 8 ? 1 : nb) * u * s * xm * 9 * 16 : 0) + nw * nmat * 64 * 16 + (norm ? nw * xm * 4 : 0);
 }
 
+// Tokens a fused-norm launch stages at m tokens (0: two token blocks, whose
+// lanes load and normalise their own fragments).
+constexpr int norm_xm(int m) { return m <= 1 ? 1 : m <= 2 ? 2 : m <= 4 ? 4 : m <= 8 ? 8 : m <= 16 ? 16 : 0; }
+// Whether a launch shape has the fused norm for that many staged tokens: above
+// four tokens a lane keeps its activations and norm weights in registers beside
+// its weight loads, which fits for at most four slots per wave (K <= 2048 with
+// eight waves, 4096 with sixteen).  The SwiGLU pair has it up to four tokens: its
+// several workgroups per CU would each repeat the norm (6 / 12 / 24 tokens cost
+// 2.9 / 5.5 / 14 us more, against 3.3 / 3.5 / 4.3 for the norm as a launch).
+constexpr bool norm_shape(int nw, int u, int nb, int nmat, bool fold, int xm) {
+  const int s = fold ? 2 : 1;
+  if (nb == 0 || (nmat == 2 && (xm == 0 || xm > 4))) return false;
+  if (xm == 0) return !fold && nw == 8 && nb == 2;
+  if (xm == 16 && fold) return false;
+  return (xm <= 4 || u * nb * s <= 4) && skinny_lds_bytes(nw, u, nb, nmat, s, xm, true) + nw * u * nb * s * 128 <= kLdsLimit;
+}
+
+// Eight bf16 activations after rms_norm with row factor r and eight norm
+// weights: bf16(w * bf16(x * r)) (engine/model.py:29-34).
+__device__ __forceinline__ u32x4 norm_piece(u32x4 xv, u32x4 g4, float r) {
+  u32x4 o;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const float x0 = bf16_bits_to_f32(static_cast<uint16_t>(xv[e])), x1 = __uint_as_float(xv[e] & 0xffff0000u);
+    const float g0 = bf16_bits_to_f32(static_cast<uint16_t>(g4[e])), g1 = __uint_as_float(g4[e] & 0xffff0000u);
+    const uint32_t n = pack_bf16x2(x0 * r, x1 * r);
+    o[e] = pack_bf16x2(g0 * bf16_bits_to_f32(static_cast<uint16_t>(n)), g1 * __uint_as_float(n & 0xffff0000u));
+  }
+  return o;
+}
+
+// RoPE of the q and k members of a q|k|v launch in its epilogue
+// (engine/model.py:53-56, 172-173): cos / sin bf16 [m, hd], or null.  Members 0
+// and 1 are then tiled by rotation pairs: tile j of a head is rows 8j .. 8j+7
+// of its first half and their partners hd/2 on.
+struct RopeArgs {
+  const uint16_t* cos;
+  const uint16_t* sin;
+  int hd;
+};
+
 // Template parameters:
 //   NW, U, NB  waves per workgroup, 64-k slots per batch, batches per wave
 //              issued at once (NB = 0: a loop over pairs of batches)
@@ -119,18 +160,20 @@ constexpr int skinny_lds_bytes(int nw, int u, int nb, int nmat, int s, int xm, b
 //              and eps (engine/model.py:29-34), computed on the staged pieces
 //              (splits == 1: the workgroup holds whole rows)
 //   TM         16-token column blocks (M <= 16 TM; 2: unfolded, direct loads)
+//   ROPE       RoPE of members 0 and 1 in the epilogue (RopeArgs; splits == 1)
 // The launcher picks one combination per call (launch_kernel); the static
 // asserts below list the combinations that exist.
-template <int NW, int U, int NB, int NMAT, bool OUT_F32, bool K64, bool FOLD, int XM, bool NORM, int TM = 1>
+template <int NW, int U, int NB, int NMAT, bool OUT_F32, bool K64, bool FOLD, int XM, bool NORM, int TM = 1, bool ROPE = false>
 __global__ __launch_bounds__(64 * NW, skinny_occ(NW, NB, NMAT, TM)) void skinny_kernel(const uint16_t* __restrict__ x, GroupArgs a, int M,
                                                          int K, int splits, float* __restrict__ partials,
                                                          unsigned long long* __restrict__ pairs,
                                                          const uint16_t* __restrict__ nw, float eps,
-                                                         unsigned long long* __restrict__ keys) {
+                                                         unsigned long long* __restrict__ keys, RopeArgs rope) {
   static_assert(!FOLD || NMAT == 1, "folding serves single matrices");
-  static_assert(XM == 0 || (NB > 0 && K64 && (8 % XM == 0 || (XM == 16 && !NORM && !FOLD))),
+  static_assert(XM == 0 || (NB > 0 && K64 && (8 % XM == 0 || (XM == 16 && !FOLD))),
                 "activation staging covers issue-once shapes");
-  static_assert(!NORM || (XM > 0 && !OUT_F32), "the fused norm works on staged activations");
+  static_assert(!NORM || (!OUT_F32 && norm_shape(NW, U, NB, NMAT, FOLD, XM)), "the fused norm's launch shapes");
+  static_assert(!ROPE || (NORM && NMAT == 1 && !FOLD), "RoPE in the epilogue of the q|k|v launch");
   static_assert(TM == 1 || (TM == 2 && !FOLD && XM == 0), "two token blocks: unfolded, direct activation loads");
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // wave-uniform: scalar loop control
@@ -152,7 +195,17 @@ __global__ __launch_bounds__(64 * NW, skinny_occ(NW, NB, NMAT, TM)) void skinny_
   const int mm = FOLD ? idx >> 3 : idx >> 4;
   const int oi = FOLD ? 8 * half + (idx & 7) : idx & 15;
   const int nout = M * (FOLD ? 8 : 16);
-  const bool has_out = idx < nout && row0 + oi < N;
+  // (ROPE) members 0 and 1: the tile's rows 0-7 are rows r0 .. r0 + 7 of a
+  // head's first half, rows 8-15 their partners half a head on
+  const bool roped = ROPE && g < 2;
+  int r0 = row0;
+  if (roped) {
+    const int tl = row0 >> 4, per = rope.hd >> 4;  // tiles per head
+    r0 = tl / per * rope.hd + tl % per * 8;
+  }
+  // output row of this thread
+  const int orow = roped ? r0 + (oi & 7) + (oi >> 3) * (rope.hd >> 1) : row0 + oi;
+  const bool has_out = idx < nout && orow < N;
 
   // (splits <= 2 and nchunks <= 2^16: 32-bit arithmetic)
   const int nchunks = (K + 63) >> 6;
@@ -170,12 +223,16 @@ __global__ __launch_bounds__(64 * NW, skinny_occ(NW, NB, NMAT, TM)) void skinny_
 #pragma unroll
   for (int mat = 0; mat < NMAT; ++mat) {
     const int8_t* qg = (NMAT == 2) ? a.q[mat] : pick_early(a.q, g);
-    wres[mat] = make_rsrc(qg + (static_cast<int64_t>(row0 >> 4) * nchunks + cb) * 1024,
-                          static_cast<int64_t>(ce - cb) * 1024);
+    // (roped: through the partners' block row; a chunk past K then reads
+    // another row's weights, which meet activations masked to zero)
+    wres[mat] = make_rsrc(qg + (static_cast<int64_t>(r0 >> 4) * nchunks + cb) * 1024,
+                          (static_cast<int64_t>(ce - cb) + (roped ? (rope.hd >> 5) * nchunks : 0)) * 1024);
   }
   // A operand row lrow: tile row lrow, or (folded) row 8 half + lrow % 8 of
-  // the slot's chunk lrow / 8
-  const int woff = FOLD ? (lrow >> 3) * 1024 + (8 * half + (lrow & 7) + 16 * kgrp) * 16 : lane * 16;
+  // the slot's chunk lrow / 8, or (roped) row lrow % 8 of the rotation pair's
+  // half lrow / 8
+  int woff = FOLD ? (lrow >> 3) * 1024 + (8 * half + (lrow & 7) + 16 * kgrp) * 16 : lane * 16;
+  if (roped) woff = (lrow >> 3) * (rope.hd >> 5) * nchunks * 1024 + ((r0 & 15) + (lrow & 7) + 16 * kgrp) * 16;
   // B operand column lrow: token min(lrow, M - 1), or (folded) token lrow % M
   // of the slot's chunk lrow / M (columns >= 2M repeat column 0, unused); this
   // lane's 16 k of the chunk
@@ -234,13 +291,13 @@ __global__ __launch_bounds__(64 * NW, skinny_occ(NW, NB, NMAT, TM)) void skinny_
       for (int mat = 0; mat < NMAT; ++mat)
         b.w[u][mat] = __builtin_amdgcn_raw_buffer_load_b128(wres[mat], woff, (c + u) * S * 1024, kLoadNT);
   };
-  auto load_batch = [&](Batch& b, int c) {
+  auto load_batch = [&](Batch& b, int c, bool weights = true) {
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       const int c0 = (c + u) * S;  // first chunk of the slot, from cb
 #pragma unroll
       for (int mat = 0; mat < NMAT; ++mat)
-        b.w[u][mat] = __builtin_amdgcn_raw_buffer_load_b128(wres[mat], woff, c0 * 1024, kLoadNT);
+        if (weights) b.w[u][mat] = __builtin_amdgcn_raw_buffer_load_b128(wres[mat], woff, c0 * 1024, kLoadNT);
       // (chunks past the range, and K % 64 != 0 columns past K, read the
       // next row or zeros; mac_batch masks them)
       b.x[u][0] = __builtin_amdgcn_raw_buffer_load_b128(xres, xoff, (cb + c0) * 128, 0);
@@ -296,15 +353,23 @@ __global__ __launch_bounds__(64 * NW, skinny_occ(NW, NB, NMAT, TM)) void skinny_
   constexpr int kStep = NW * U;
   const int first = wave * U;
   // epilogue operands (clamped to a valid output, so the loads need no branch)
-  auto load_epi = [&] { return epilogue_load<NMAT>(a, g, min(row0 + oi, N - 1), min(mm, M - 1), N, x); };
+  auto load_epi = [&] { return epilogue_load<NMAT>(a, g, min(orow, N - 1), min(mm, M - 1), N, x); };
   EpiIn<NMAT> epi;
+  uint16_t rc = 0, rs = 0;  // (ROPE) cos and sin of this thread's token and dimension
   if constexpr (NB > 0) {
     Batch bt[NB];
     u32x4 xpiece[XM > 0 ? XPASS : 1];
-    u32x4 wpiece[NORM ? XPASS : 1];  // NORM: the norm weights of the same columns
+    // NORM: the norm weights of the same columns in registers, or (above four
+    // staged tokens, and with two token blocks) the workgroup's in LDS
+    constexpr bool NWL = NORM && (XM == 0 || XM >= 8);
+    constexpr int NP = NWL ? NW * U * NB * S * 8 : 1;  // 16-byte pieces of the chunks covered
+    static_assert(NP <= 64 * NW, "one piece per thread");
+    __shared__ u32x4 nwst[NP];
+    u32x4 wpiece[NORM && !NWL ? XPASS : 1];
+    const __amdgpu_buffer_rsrc_t nres = make_rsrc(NORM ? nw : x, NORM ? static_cast<int64_t>(K) * 2 : 0);
+    if constexpr (NWL) wpiece[0] = __builtin_amdgcn_raw_buffer_load_b128(nres, idx * 16, 0, 0);
     if constexpr (XM > 0) {
       // the pieces first, so that parking them waits for them alone
-      const __amdgpu_buffer_rsrc_t nres = make_rsrc(NORM ? nw : x, NORM ? static_cast<int64_t>(K) * 2 : 0);
 #pragma unroll
       for (int i = 0; i < XPASS; ++i) {
         const int p = lane + 64 * i;
@@ -320,9 +385,16 @@ __global__ __launch_bounds__(64 * NW, skinny_occ(NW, NB, NMAT, TM)) void skinny_
         const bool in = p < XP && ch < ce;
         const int off = in ? t * K * 2 + ch * 128 + (p & 7) * 16 : 0x7ffffff0;
         xpiece[i] = __builtin_amdgcn_raw_buffer_load_b128(xres, off, 0, 0);
-        if constexpr (NORM)
+        if constexpr (NORM && !NWL)
           wpiece[i] = __builtin_amdgcn_raw_buffer_load_b128(nres, in ? ch * 128 + (p & 7) * 16 : 0x7ffffff0, 0, 0);
       }
+#pragma unroll
+      for (int j = 0; j < NB; ++j) load_w(bt[j], first + j * kStep);
+    } else if constexpr (NORM) {
+      // the activations first: the norm waits for them alone
+#pragma unroll
+      for (int j = 0; j < NB; ++j) load_batch(bt[j], first + j * kStep, false);
+      __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int j = 0; j < NB; ++j) load_w(bt[j], first + j * kStep);
     } else {
@@ -330,46 +402,119 @@ __global__ __launch_bounds__(64 * NW, skinny_occ(NW, NB, NMAT, TM)) void skinny_
       for (int j = 0; j < NB; ++j) load_batch(bt[j], first + j * kStep);
     }
     epi = load_epi();  // behind the weight loads
+    if constexpr (ROPE) {
+      const int64_t at = static_cast<int64_t>(min(mm, M - 1)) * rope.hd + (roped ? orow % rope.hd : 0);
+      rc = rope.cos[at];
+      rs = rope.sin[at];
+    }
     __builtin_amdgcn_sched_barrier(0);  // every load issued before the first wait
-    if constexpr (NORM) {
+    if constexpr (NORM && XM == 0) {
+      // Two token blocks: a lane holds tokens min(lrow, M - 1) and min(16 +
+      // lrow, M - 1), 16 k of each of its chunks.  The same formula as below on
+      // those fragments: sums of squares over the lane's chunks, the four k
+      // groups by a butterfly, the waves in order through LDS; the norm
+      // weights come from LDS.
+      __shared__ float npart2[NW][16 * TM];
+      if (idx < NP) nwst[idx] = wpiece[0];
+      float ss[TM], r[TM];
+#pragma unroll
+      for (int t = 0; t < TM; ++t) ss[t] = 0.f;
+#pragma unroll
+      for (int j = 0; j < NB; ++j)
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          // (a chunk past K is the next token's: masked)
+          const uint32_t mask = first + j * kStep + u < ce ? 0xffffffffu : 0u;
+#pragma unroll
+          for (int f = 0; f < 2 * TM; ++f) {
+            bt[j].x[u][f] &= mask;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+              const float lo = bf16_bits_to_f32(static_cast<uint16_t>(bt[j].x[u][f][e]));
+              const float hi = __uint_as_float(bt[j].x[u][f][e] & 0xffff0000u);
+              ss[f >> 1] += lo * lo;
+              ss[f >> 1] += hi * hi;
+            }
+          }
+        }
+#pragma unroll
+      for (int t = 0; t < TM; ++t) {
+        ss[t] += __shfl_xor(ss[t], 16);
+        ss[t] += __shfl_xor(ss[t], 32);
+        if (kgrp == 0) npart2[wave][16 * t + lrow] = ss[t];
+      }
+      __syncthreads();
+#pragma unroll
+      for (int t = 0; t < TM; ++t) {
+        float tot = 0.f;
+#pragma unroll
+        for (int w = 0; w < NW; ++w) tot += npart2[w][16 * t + lrow];
+        r[t] = 1.0f / sqrtf(tot / static_cast<float>(K) + eps);
+      }
+#pragma unroll
+      for (int j = 0; j < NB; ++j)
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+#pragma unroll
+          for (int hf = 0; hf < 2; ++hf) {
+            const u32x4 g4 = nwst[(first + j * kStep + u) * 8 + kgrp * 2 + hf];
+#pragma unroll
+            for (int t = 0; t < TM; ++t)
+              bt[j].x[u][2 * t + hf] = norm_piece(bt[j].x[u][2 * t + hf], g4, r[t]);
+          }
+    }
+    if constexpr (NORM && XM > 0) {
       // rms_norm on the staged pieces.  All pieces of a lane belong to token
-      // (lane / 8) % XM (XM divides 8).  Sum of squares in a fixed order:
-      // each lane over its pieces, the lanes of a token by a butterfly, the
-      // waves in order through LDS; then r = 1 / sqrt(mean + eps) and
-      // h = bf16(w * bf16(x * r)), the reference's roundings.
-      const int tl = (lane >> 3) % XM;
-      float ss = 0.f;
+      // (lane / 8) % XM (XM divides 8), with sixteen tokens the pieces of even
+      // passes to token lane / 8 and those of odd passes to 8 + lane / 8.  Sum
+      // of squares in a fixed order: each lane over its pieces, the lanes of a
+      // token by a butterfly, the waves in order through LDS; then
+      // r = 1 / sqrt(mean + eps) and h = bf16(w * bf16(x * r)), the
+      // reference's roundings.
+      constexpr int TL = XM == 16 ? 2 : 1;  // tokens per lane
+      const int tl0 = (lane >> 3) % XM;
+      float ss[TL], rr[TL];
+#pragma unroll
+      for (int t = 0; t < TL; ++t) ss[t] = 0.f;
 #pragma unroll
       for (int i = 0; i < XPASS; ++i)
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
           const float lo = bf16_bits_to_f32(static_cast<uint16_t>(xpiece[i][e]));
           const float hi = bf16_bits_to_f32(static_cast<uint16_t>(xpiece[i][e] >> 16));
-          ss += lo * lo;
-          ss += hi * hi;
+          ss[i % TL] += lo * lo;
+          ss[i % TL] += hi * hi;
         }
-#pragma unroll
-      for (int off = 1; off < 64; off <<= 1)
-        if ((off >> 3) % XM == 0 || off < 8) ss += __shfl_xor(ss, off);  // lanes of the same token
       __shared__ float npart[NW][XM];
-      if ((lane & ~(8 * XM - 1) & ~7) == 0 && (lane & 7) == 0) npart[wave][tl] = ss;
-      __syncthreads();
-      float tot = 0.f;
+      if constexpr (NWL)
+        if (idx < NP) nwst[idx] = wpiece[0];
 #pragma unroll
-      for (int w = 0; w < NW; ++w) tot += npart[w][tl];
-      const float r = 1.0f / sqrtf(tot / static_cast<float>(K) + eps);
+      for (int t = 0; t < TL; ++t) {
+#pragma unroll
+        for (int off = 1; off < 64; off <<= 1)
+          if (off < 8 || (off >> 3) % XM == 0) ss[t] += __shfl_xor(ss[t], off);  // lanes of the same token
+        if ((lane & ~(8 * XM - 1) & ~7) == 0 && (lane & 7) == 0) npart[wave][tl0 + 8 * t] = ss[t];
+      }
+      __syncthreads();
+#pragma unroll
+      for (int t = 0; t < TL; ++t) {
+        float tot = 0.f;
+#pragma unroll
+        for (int w = 0; w < NW; ++w) tot += npart[w][tl0 + 8 * t];
+        rr[t] = 1.0f / sqrtf(tot / static_cast<float>(K) + eps);
+      }
 #pragma unroll
       for (int i = 0; i < XPASS; ++i) {
-        u32x4 o;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const float x0 = bf16_bits_to_f32(static_cast<uint16_t>(xpiece[i][e]));
-          const float x1 = bf16_bits_to_f32(static_cast<uint16_t>(xpiece[i][e] >> 16));
-          const float g0 = bf16_bits_to_f32(static_cast<uint16_t>(wpiece[i][e]));
-          const float g1 = bf16_bits_to_f32(static_cast<uint16_t>(wpiece[i][e] >> 16));
-          o[e] = pack_bf16x2(g0 * bf16_bits_to_f32(f32_to_bf16_bits(x0 * r)),
-                             g1 * bf16_bits_to_f32(f32_to_bf16_bits(x1 * r)));
+        const float r = rr[i % TL];
+        const int tl = tl0 + 8 * (i % TL);
+        u32x4 gw;
+        if constexpr (NWL) {
+          const int p = lane + 64 * i, cr = p / (8 * XM), sw = cr / S;
+          gw = nwst[((first + (sw / U) * kStep + sw % U) * S + cr % S) * 8 + (p & 7)];
+        } else {
+          gw = wpiece[i];
         }
+        const u32x4 o = norm_piece(xpiece[i], gw, r);
         xpiece[i] = tl < M ? o : u32x4{0u, 0u, 0u, 0u};  // (tokens past M: never read)
       }
     }
@@ -470,6 +615,21 @@ __global__ __launch_bounds__(64 * NW, skinny_occ(NW, NB, NMAT, TM)) void skinny_
       return;
     }
   }
+  if constexpr (ROPE) {
+    // the bf16 projection, then the rotation's three bf16 roundings; the
+    // partner dimension is the output of thread idx ^ 8, in the same wave
+    if (roped) {
+      float out = v[0] * epi.s[0];
+      if (pick_early(a.bias, g)) out += bf16_bits_to_f32(epi.bias);
+      out = bf16_bits_to_f32(f32_to_bf16_bits(out));
+      const float other = __shfl_xor(out, 8);
+      const float c = bf16_bits_to_f32(rc), sn = bf16_bits_to_f32(rs);
+      const float o = bf16_bits_to_f32(f32_to_bf16_bits(out * c)) +
+                      bf16_bits_to_f32(f32_to_bf16_bits((oi < 8 ? -other : other) * sn));
+      if (live && has_out) store_out<false>(pick_early(a.y, g), static_cast<int64_t>(mm) * N + orow, o);
+      return;
+    }
+  }
   if (!live) return;
   if (NMAT == 1 && pairs) {
     // The two K halves of this tile meet in one 64-bit slot per output.
@@ -485,14 +645,14 @@ __global__ __launch_bounds__(64 * NW, skinny_occ(NW, NB, NMAT, TM)) void skinny_
     if (prev >> 32) {
       __hip_atomic_exchange(slot, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
       v[0] += __uint_as_float(static_cast<uint32_t>(prev));
-      if (has_out) epilogue<NMAT, OUT_F32>(a, g, row0 + oi, mm, N, v, epi);
+      if (has_out) epilogue<NMAT, OUT_F32>(a, g, orow, mm, N, v, epi);
     }
   } else if (splits > 1) {
     float* mine = partials + (static_cast<int64_t>(tile) * splits + s) * (NMAT * 256 * TM);
 #pragma unroll
     for (int mat = 0; mat < NMAT; ++mat) mine[mat * 256 * TM + idx] = v[mat];
   } else if (has_out) {
-    epilogue<NMAT, OUT_F32>(a, g, row0 + oi, mm, N, v, epi);
+    epilogue<NMAT, OUT_F32>(a, g, orow, mm, N, v, epi);
   }
 }
 
@@ -525,15 +685,29 @@ __global__ __launch_bounds__(256) void skinny_reduce_kernel(GroupArgs a, int M, 
 
 // Launches one skinny_kernel instance (and records it for pgs_last_plan:
 // this function's pretty name spells out the instance's template arguments).
-template <int NW, int U, int NB, int NMAT, bool OUT_F32, bool K64, bool FOLD, int XM, bool NORM, int TM = 1>
+template <int NW, int U, int NB, int NMAT, bool OUT_F32, bool K64, bool FOLD, int XM, bool NORM, int TM = 1, bool ROPE = false>
 int launch_instance(Problem& p, const SkinnyPlan& plan, hipStream_t st) {
   const int64_t grid = static_cast<int64_t>(plan.tiles) * (FOLD ? 2 : plan.splits);
   unsigned long long* pairs = plan.pair ? p.pairs : nullptr;
   note_launch(__PRETTY_FUNCTION__, grid, plan.splits, plan.splits > 1 && !plan.pair ? "skinny_reduce_kernel" : nullptr);
-  hipLaunchKernelGGL((skinny_kernel<NW, U, NB, NMAT, OUT_F32, K64, FOLD, XM, NORM, TM>), dim3(static_cast<unsigned>(grid)),
+  hipLaunchKernelGGL((skinny_kernel<NW, U, NB, NMAT, OUT_F32, K64, FOLD, XM, NORM, TM, ROPE>), dim3(static_cast<unsigned>(grid)),
                      dim3(64 * NW), 0, st, p.x, p.args, p.m, p.k, plan.splits, p.partials, pairs, p.norm_w, p.eps,
-                     p.keys);
+                     p.keys, RopeArgs{p.rope_cos, p.rope_sin, p.rope_hd});
   return check_launch("w8a16 skinny kernel");
+}
+
+// The fused-norm instance for XM staged tokens (0: two token blocks).
+template <int NW, int U, int NB, int NMAT, bool FOLD, int XM>
+int launch_norm(Problem& p, const SkinnyPlan& plan, hipStream_t st) {
+  if constexpr (norm_shape(NW, U, NB, NMAT, FOLD, XM)) {
+    constexpr int TM = XM == 0 ? 2 : 1;
+    if constexpr (NMAT == 1 && !FOLD)
+      if (p.rope_cos) return launch_instance<NW, U, NB, NMAT, false, true, FOLD, XM, true, TM, true>(p, plan, st);
+    if (p.rope_cos) return fail(PGS_ERR_INVALID_ARGUMENT, "w8a16 skinny: no RoPE in this launch");
+    return launch_instance<NW, U, NB, NMAT, false, true, FOLD, XM, true, TM>(p, plan, st);
+  } else {
+    return fail(PGS_ERR_INVALID_ARGUMENT, "w8a16 skinny: no fused norm for this launch shape (m=%d)", p.m);
+  }
 }
 
 template <int NW, int U, int NB, int NMAT, bool OUT_F32, bool FOLD>
@@ -541,14 +715,16 @@ int launch_kernel(Problem& p, const SkinnyPlan& plan, hipStream_t st) {
   if constexpr (NB > 0 && !OUT_F32) {
     // rms_norm applied to the staged activations
     if (p.norm_w) {
-      if (p.k % 64 != 0 || p.m > 4 || plan.splits != 1 || plan.pair)
-        return fail(PGS_ERR_INVALID_ARGUMENT, "w8a16 skinny: the fused norm needs m <= 4 and one K range");
-      constexpr int S = FOLD ? 2 : 1;
-      if (p.m == 1) return launch_instance<NW, U, NB, NMAT, OUT_F32, true, FOLD, 1, true>(p, plan, st);
-      if (p.m == 2) return launch_instance<NW, U, NB, NMAT, OUT_F32, true, FOLD, 2, true>(p, plan, st);
-      if constexpr (skinny_lds_bytes(NW, U, NB, NMAT, S, 4, true) <= kLdsLimit)
-        return launch_instance<NW, U, NB, NMAT, OUT_F32, true, FOLD, 4, true>(p, plan, st);
-      return fail(PGS_ERR_INVALID_ARGUMENT, "w8a16 skinny: the fused norm's staging exceeds LDS");
+      if (p.k % 64 != 0 || plan.splits != 1 || plan.pair)
+        return fail(PGS_ERR_INVALID_ARGUMENT, "w8a16 skinny: the fused norm needs K %% 64 == 0 and one K range");
+      switch (norm_xm(p.m)) {
+        case 1: return launch_norm<NW, U, NB, NMAT, FOLD, 1>(p, plan, st);
+        case 2: return launch_norm<NW, U, NB, NMAT, FOLD, 2>(p, plan, st);
+        case 4: return launch_norm<NW, U, NB, NMAT, FOLD, 4>(p, plan, st);
+        case 8: return launch_norm<NW, U, NB, NMAT, FOLD, 8>(p, plan, st);
+        case 16: return launch_norm<NW, U, NB, NMAT, FOLD, 16>(p, plan, st);
+        default: return launch_norm<NW, U, NB, NMAT, FOLD, 0>(p, plan, st);
+      }
     }
   }
   if (p.norm_w) return fail(PGS_ERR_INVALID_ARGUMENT, "w8a16 skinny: the fused norm needs a bf16 output");
@@ -656,23 +832,25 @@ int launch_shape(Problem& p, const SkinnyPlan& plan, hipStream_t st) {
   }
 }
 
-// The SwiGLU pair at 14..16 tokens with a short K (K % 64 == 0, at most
-// NW * CPW chunks): RT row tiles per workgroup instead of one.  With one
-// tile per workgroup every workgroup loads the tokens' whole activation
-// rows for its 16 rows, as many bytes as its weights, and at 16 tokens each
-// of those loads touches 16 rows; here each activation fragment feeds the
-// RT tiles' gate and up MFMAs, and RT = 3 gives ceil(688 / 3) = 230
-// workgroups for an 11008-row pair, at most one per CU and at most 48 rows
-// per CU as before.  Wave w takes chunks w * CPW .. w * CPW + CPW - 1 of
-// every tile and issues all of its loads at once (one memory round trip);
-// the waves' partial tiles are summed through LDS in wave order (a fixed
-// order: reproducible), then each output thread applies silu(g s_g)(u s_u)
-// (engine/model.py:188-189).  Measured on the 11008 x 2048 pair (graphs over
-// 36 layers, us, one-tile plan -> this kernel): 16 tokens 11.56 -> 11.20,
-// 15: 11.36 -> 11.24, 14: 11.15 -> 11.02, but 13: 11.0 -> 11.1, 12: 10.8 ->
-// 10.9 and 9: 10.1 -> 10.5, hence 14..16 tokens; 8 waves x 4 chunks (11.9),
-// four tiles per workgroup (11.9) and two (13.0) are slower at 16 tokens.
-template <int RT, int NW, int CPW>
+// The SwiGLU pair at 14..32 tokens with a short K (K % 64 == 0, at most
+// NW * CPW chunks): RT row tiles per workgroup instead of one.  With one tile
+// per workgroup every workgroup loads the tokens'
+// whole activation rows for its 16 rows, as many bytes as its weights at 16
+// tokens and twice as many at 32; here each activation fragment feeds the RT
+// tiles' gate and up MFMAs, and RT = ceil(tiles / 256) gives at most one
+// workgroup per CU (230 for an 11008-row pair).  Wave w takes chunks w * CPW ..
+// w * CPW + CPW - 1 of every tile and issues all of its loads at once (one
+// memory round trip), the activations first; the waves' partial tiles are
+// summed through LDS in wave order (a fixed order: reproducible), then each
+// output thread applies silu(g s_g)(u s_u) (engine/model.py:188-189).
+// Measured on the 11008 x 2048 pair (us, one-tile plan -> this kernel): 16
+// tokens 11.56 -> 11.20, 14: 11.15 -> 11.02, but 13: 11.0 -> 11.1 and 9: 10.1 ->
+// 10.5 (sixteen waves of two chunks); two token blocks (eight waves of four
+// chunks, so that a lane's loads fit its registers) 24: 14.7 -> 14.0, 32 tokens
+// 1.2 us less; the 4864 x 896 pair at 20 tokens 9.5 -> 6.3 (two tiles).  The
+// norm in front of it here cost 2.6 (6 tokens) to 4.9 us (24), as much as its
+// launch: the widening waits for it, so the pair has no fused norm.
+template <int RT, int NW, int CPW, int TM>
 __global__ __launch_bounds__(64 * NW, 1) void pair_tiles_kernel(const uint16_t* __restrict__ x, GroupArgs a, int M,
                                                                 int K, int tiles) {
   const int lane = threadIdx.x & 63;
@@ -681,6 +859,7 @@ __global__ __launch_bounds__(64 * NW, 1) void pair_tiles_kernel(const uint16_t* 
   const int N = a.n[0];
   const int nchunks = K >> 6;
   const int t0 = blockIdx.x * RT;
+  const int idx = threadIdx.x;
   // one buffer resource per tile and matrix over the tile's whole block
   // row; a tile past the last reads zeros without touching memory
   __amdgpu_buffer_rsrc_t wres[RT][2];
@@ -693,82 +872,130 @@ __global__ __launch_bounds__(64 * NW, 1) void pair_tiles_kernel(const uint16_t* 
                                ok ? static_cast<int64_t>(nchunks) * 1024 : 0);
     }
   const __amdgpu_buffer_rsrc_t xres = make_rsrc(x, static_cast<int64_t>(M) * K * 2);
-  // B operand column lrow: token min(lrow, M - 1); this lane's 16 k of the chunk
-  const int xoff = min(lrow, M - 1) * K * 2 + kgrp * 32;
-
-  // output of this thread: tile er, token mm, tile row oi; its scales are
-  // requested first, from a clamped (valid) row, so no branch waits for them
-  const int idx = threadIdx.x;
-  const int er = min(idx >> 8, RT - 1), mm = (idx >> 4) & 15, oi = idx & 15;
-  const int row = (t0 + er) * 16 + oi;
-  const bool has_out = idx < 256 * RT && mm < M && row < N;
-  const int crow = min(row, N - 1);
-  const float sg = a.scale[0][crow], su = a.scale[1][crow];
-
-  u32x4 w[CPW][RT][2], xb[CPW][2];
+  // B operand column lrow of block t: token min(16 t + lrow, M - 1); this lane's 16 k of the chunk
+  int xoff[TM];
 #pragma unroll
-  for (int j = 0; j < CPW; ++j) {
-    const int c = wave * CPW + j;
+  for (int t = 0; t < TM; ++t) xoff[t] = min(16 * t + lrow, M - 1) * K * 2 + kgrp * 32;
+
+  // outputs of this thread: o = idx, idx + 64 NW, ... of [tile][token][row of
+  // the tile]; their scales are requested behind the weights, from clamped
+  // (valid) rows, so no branch waits for them
+  constexpr int OPT = (RT * TM * 256 + 64 * NW - 1) / (64 * NW);
+  float sg[OPT], su[OPT];
+  auto out_row = [&](int o) { return (t0 + o / (256 * TM)) * 16 + (o & 15); };
+  auto load_scales = [&] {
+#pragma unroll
+    for (int i = 0; i < OPT; ++i) {
+      const int crow = min(out_row(idx + i * 64 * NW), N - 1);
+      sg[i] = a.scale[0][crow];
+      su[i] = a.scale[1][crow];
+    }
+  };
+  u32x4 w[CPW][RT][2], xb[CPW][TM][2];
+#pragma unroll
+  for (int j = 0; j < CPW; ++j)
+#pragma unroll
+    for (int t = 0; t < TM; ++t) {
+      xb[j][t][0] = __builtin_amdgcn_raw_buffer_load_b128(xres, xoff[t], (wave * CPW + j) * 128, 0);
+      xb[j][t][1] = __builtin_amdgcn_raw_buffer_load_b128(xres, xoff[t] + 16, (wave * CPW + j) * 128, 0);
+    }
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int j = 0; j < CPW; ++j)
 #pragma unroll
     for (int r = 0; r < RT; ++r)
 #pragma unroll
       for (int mat = 0; mat < 2; ++mat)
-        w[j][r][mat] = __builtin_amdgcn_raw_buffer_load_b128(wres[r][mat], lane * 16, c * 1024, kLoadNT);
-    xb[j][0] = __builtin_amdgcn_raw_buffer_load_b128(xres, xoff, c * 128, 0);
-    xb[j][1] = __builtin_amdgcn_raw_buffer_load_b128(xres, xoff + 16, c * 128, 0);
-  }
-  f32x4 acc[RT][2];
-#pragma unroll
-  for (int r = 0; r < RT; ++r) acc[r][0] = acc[r][1] = f32x4{0.f, 0.f, 0.f, 0.f};
+        w[j][r][mat] = __builtin_amdgcn_raw_buffer_load_b128(wres[r][mat], lane * 16, (wave * CPW + j) * 1024, kLoadNT);
+  __builtin_amdgcn_sched_barrier(0);  // every load issued before the first wait
+  // a chunk past K reads zero weights; its activations (the next token's
+  // row, or zeros) are masked too, so non-finite values cannot leak in
 #pragma unroll
   for (int j = 0; j < CPW; ++j) {
-    // a chunk past K reads zero weights; its activations (the next token's
-    // row, or zeros) are masked too, so non-finite values cannot leak in
     const uint32_t mask = wave * CPW + j < nchunks ? 0xffffffffu : 0u;
-    const bf16x8 b0 = __builtin_bit_cast(bf16x8, xb[j][0] & mask);
-    const bf16x8 b1 = __builtin_bit_cast(bf16x8, xb[j][1] & mask);
+#pragma unroll
+    for (int t = 0; t < TM; ++t) {
+      xb[j][t][0] &= mask;
+      xb[j][t][1] &= mask;
+    }
+  }
+  load_scales();
+  f32x4 acc[RT][2][TM];
+#pragma unroll
+  for (int r = 0; r < RT; ++r)
+#pragma unroll
+    for (int mat = 0; mat < 2; ++mat)
+#pragma unroll
+      for (int t = 0; t < TM; ++t) acc[r][mat][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int j = 0; j < CPW; ++j)
 #pragma unroll
     for (int r = 0; r < RT; ++r)
 #pragma unroll
       for (int mat = 0; mat < 2; ++mat) {
-        acc[r][mat] = mfma16x16x32(i8x8_to_bf16x8(w[j][r][mat][0], w[j][r][mat][1]), b0, acc[r][mat]);
-        acc[r][mat] = mfma16x16x32(i8x8_to_bf16x8(w[j][r][mat][2], w[j][r][mat][3]), b1, acc[r][mat]);
+        const bf16x8 a0 = i8x8_to_bf16x8(w[j][r][mat][0], w[j][r][mat][1]);
+        const bf16x8 a1 = i8x8_to_bf16x8(w[j][r][mat][2], w[j][r][mat][3]);
+#pragma unroll
+        for (int t = 0; t < TM; ++t) {
+          acc[r][mat][t] = mfma16x16x32(a0, __builtin_bit_cast(bf16x8, xb[j][t][0]), acc[r][mat][t]);
+          acc[r][mat][t] = mfma16x16x32(a1, __builtin_bit_cast(bf16x8, xb[j][t][1]), acc[r][mat][t]);
+        }
+        if constexpr (TM == 2) __builtin_amdgcn_sched_barrier(0);  // (one widened operand pair at a time: registers)
       }
-  }
-  __shared__ f32x4 part[NW][RT][2][64];
+  __shared__ f32x4 part[NW][RT][2][TM][64];
 #pragma unroll
   for (int r = 0; r < RT; ++r)
 #pragma unroll
-    for (int mat = 0; mat < 2; ++mat) part[wave][r][mat][lane] = acc[r][mat];
+    for (int mat = 0; mat < 2; ++mat)
+#pragma unroll
+      for (int t = 0; t < TM; ++t) part[wave][r][mat][t][lane] = acc[r][mat][t];
   __syncthreads();
-  if (has_out) {
+#pragma unroll
+  for (int i = 0; i < OPT; ++i) {
+    const int o = idx + i * 64 * NW;
+    const int er = o / (256 * TM), mm = (o >> 4) % (16 * TM), oi = o & 15, row = out_row(o);
+    if (er >= RT || mm >= M || row >= N) continue;
     // output (row oi, token mm) of a 16x16 tile: lane acc_lane(oi, mm), register oi % 4
-    const int ln = acc_lane(oi, mm), rg = oi & 3;
+    const int ln = acc_lane(oi, mm & 15), rg = oi & 3;
     float g = 0.f, u = 0.f;
 #pragma unroll
     for (int wv = 0; wv < NW; ++wv) {
-      g += part[wv][er][0][ln][rg];
-      u += part[wv][er][1][ln][rg];
+      g += part[wv][er][0][mm >> 4][ln][rg];
+      u += part[wv][er][1][mm >> 4][ln][rg];
     }
-    store_out<false>(a.y[0], static_cast<int64_t>(mm) * N + row, silu_f32(g * sg) * (u * su));
+    store_out<false>(a.y[0], static_cast<int64_t>(mm) * N + row, silu_f32(g * sg[i]) * (u * su[i]));
   }
 }
 
-constexpr int kPairRT = 3, kPairNW = 16, kPairCPW = 2;
-
-// whether pair_tiles_kernel takes a SwiGLU pair launch
-bool pair_tiles_fits(const Problem& p, const SkinnyPlan& plan) {
-  return p.nmat == 2 && !p.out_f32 && !p.norm_w && plan.tm == 1 && plan.splits == 1 && p.m >= 14 && p.m <= 16 &&
-         p.k % 64 == 0 && p.k / 64 <= kPairNW * kPairCPW;
+// The launch of pair_tiles_kernel a SwiGLU pair takes at these sizes: row
+// tiles per workgroup (0: none), waves and chunks per wave.  Two token blocks
+// only where one round of workgroups fills more than half of the CUs.
+struct PairTiles {
+  int rt, nw, cpw;
+};
+PairTiles pair_tiles(int m, int k, const SkinnyPlan& plan) {
+  if (plan.splits != 1 || k % 64 != 0 || k > 2048) return {0, 0, 0};
+  if (m < 14 || m > 32) return {0, 0, 0};
+  if (m > 16 && (plan.tiles <= 256 || plan.tiles > 768)) return {0, 0, 0};
+  const int rt = plan.tiles > 256 && plan.tiles <= 512 ? 2 : 3;
+  if (k <= 1024) return {rt, 8, 2};
+  return m <= 16 ? PairTiles{rt, 16, 2} : PairTiles{rt, 8, 4};
 }
 
-template <int RT, int NW, int CPW>
+template <int RT, int NW, int CPW, int TM>
 int launch_pair_tiles(Problem& p, const SkinnyPlan& plan, hipStream_t st) {
   const int64_t grid = (static_cast<int64_t>(plan.tiles) + RT - 1) / RT;
   note_launch(__PRETTY_FUNCTION__, grid, 1, nullptr);
-  hipLaunchKernelGGL((pair_tiles_kernel<RT, NW, CPW>), dim3(static_cast<unsigned>(grid)), dim3(64 * NW), 0, st,
+  hipLaunchKernelGGL((pair_tiles_kernel<RT, NW, CPW, TM>), dim3(static_cast<unsigned>(grid)), dim3(64 * NW), 0, st,
                      p.x, p.args, p.m, p.k, plan.tiles);
   return check_launch("w8a16 pair tiles kernel");
+}
+
+template <int RT>
+int launch_pair(Problem& p, const PairTiles& pt, const SkinnyPlan& plan, hipStream_t st) {
+  if (p.m <= 16)
+    return pt.nw == 16 ? launch_pair_tiles<RT, 16, 2, 1>(p, plan, st) : launch_pair_tiles<RT, 8, 2, 1>(p, plan, st);
+  return pt.cpw == 4 ? launch_pair_tiles<RT, 8, 4, 2>(p, plan, st) : launch_pair_tiles<RT, 8, 2, 2>(p, plan, st);
 }
 
 }  // namespace
@@ -829,10 +1056,13 @@ SkinnyPlan plan_skinny(int m, int k, int nmat, int tiles, bool can_split) {
 }
 
 bool skinny_norm_fusable(const SkinnyPlan& p, int m, int k, bool out_f32, int nmat) {
-  if (out_f32 || m < 1 || m > 4 || k % 64 != 0 || p.splits != 1 || p.pair || p.shape == kLoopShape) return false;
+  if (out_f32 || m < 1 || m > 32 || k % 64 != 0 || p.splits != 1 || p.pair) return false;
   const SkinnyShape& sh = kSkinnyShapes[p.shape];
-  return sh.nb > 0 && skinny_lds_bytes(sh.nw, sh.u, sh.nb, nmat, p.fold ? 2 : 1, m == 1 ? 1 : m == 2 ? 2 : 4, true) <=
-                          kLdsLimit;
+  return norm_shape(sh.nw, sh.u, sh.nb, nmat, p.fold, norm_xm(m));
+}
+
+bool skinny_rope_fusable(const SkinnyPlan& p, int hd, const GroupArgs& a) {
+  return !p.fold && hd % 32 == 0 && a.n_outs == 3 && a.n[0] % hd == 0 && a.n[1] % hd == 0;
 }
 
 int64_t skinny_grid(const SkinnyPlan& p) { return static_cast<int64_t>(p.tiles) * (p.fold ? 2 : p.splits); }
@@ -848,7 +1078,10 @@ int launch_skinny(Problem& p, const SkinnyPlan& plan, hipStream_t st) {
     return fail(PGS_ERR_INVALID_ARGUMENT, "w8a16 skinny: paired split without pair slots");
   if (plan.splits > 1 && !plan.pair && (!p.partials || p.partial_bytes < skinny_partial_bytes(plan, p.nmat)))
     return fail(PGS_ERR_INVALID_ARGUMENT, "w8a16 skinny: split-K plan without a large enough workspace");
-  if (pair_tiles_fits(p, plan)) return launch_pair_tiles<kPairRT, kPairNW, kPairCPW>(p, plan, st);
+  if (p.nmat == 2 && !p.out_f32 && !p.norm_w) {
+    const PairTiles pt = pair_tiles(p.m, p.k, plan);
+    if (pt.rt) return pt.rt == 2 ? launch_pair<2>(p, pt, plan, st) : launch_pair<3>(p, pt, plan, st);
+  }
   if (p.nmat == 2) return launch_shape<2, false>(p, plan, st);
   return p.out_f32 ? launch_shape<1, true>(p, plan, st) : launch_shape<1, false>(p, plan, st);
 }

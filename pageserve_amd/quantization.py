@@ -559,10 +559,10 @@ def linear_group(x: torch.Tensor, weights: list["QuantizedWeight"], biases: list
 def rmsnorm_linear_group(x: torch.Tensor, norm_weight: torch.Tensor, eps: float, weights: list["QuantizedWeight"],
                          biases: list | None = None, out_dtype: torch.dtype = torch.bfloat16) -> list[torch.Tensor]:
     """``h = rms_norm(x, norm_weight, eps)`` then the projections of ``h``
-    (engine/model.py:166-170), in one launch for up to 4 tokens (the kernel
-    normalises the activations it stages; its fixed-order sum of squares may
-    make ``h`` differ from :func:`rmsnorm` in the last bf16 bit), otherwise
-    :func:`rmsnorm` then :func:`linear_group`."""
+    (engine/model.py:166-170), in one launch for up to 32 tokens (above 4 of
+    them for K up to 2048; the kernel normalises the activations it loads; its
+    fixed-order sum of squares may make ``h`` differ from :func:`rmsnorm` in
+    the last bf16 bit), otherwise :func:`rmsnorm` then :func:`linear_group`."""
     return _linear_group(x, weights, biases, out_dtype, norm_weight, eps)
 
 
@@ -587,6 +587,23 @@ def _linear_group(x, weights, biases, out_dtype, norm_weight, eps) -> list[torch
                                       eps, ws, ws_bytes)
 
 
+def _rmsnorm_qkv_rope(x, norm_weight, eps, weights, biases, cos, sin, head_dim) -> list[torch.Tensor]:
+    """:func:`rmsnorm_linear_group` of q, k and v, then :func:`rope_qk` of the
+    first two (engine/model.py:166-173), in one launch where the norm runs
+    inside the projection and the heads allow it.  ``q`` and ``k`` must be
+    whole heads of ``head_dim``."""
+    ops = [w._launch_operands() for w in weights]
+    _, _, _, k, dev = ops[0]
+    if any(o[3] != k or o[4] != dev for o in ops):
+        raise ValueError("linear_group: weights must share device and in_features")
+    m = x.numel() // k if k else 0
+    c, s = _rope_tables(cos, sin, m, head_dim, dev)
+    qs, ss, ns = [o[0] for o in ops], [o[1] for o in ops], tuple(o[2] for o in ops)
+    ws, ws_bytes, _buf = _ws_args(dev, x, k, ns, False, True)
+    return _native.load_host().qkv_rope(x, qs, ss, list(biases) if biases is not None else [None] * 3, ns, k,
+                                        norm_weight, eps, c, s, head_dim, ws, ws_bytes)
+
+
 def swiglu(x: torch.Tensor, gate: "QuantizedWeight", up: "QuantizedWeight") -> torch.Tensor:
     """``F.silu(F.linear(x, gate)) * F.linear(x, up)`` in one launch
     (engine/model.py:188-190); fp32 inside, one rounding to bf16."""
@@ -596,7 +613,7 @@ def swiglu(x: torch.Tensor, gate: "QuantizedWeight", up: "QuantizedWeight") -> t
 def rmsnorm_swiglu(x: torch.Tensor, norm_weight: torch.Tensor, eps: float, gate: "QuantizedWeight",
                    up: "QuantizedWeight") -> torch.Tensor:
     """``h = rms_norm(x, norm_weight, eps)`` then :func:`swiglu` of ``h``
-    (engine/model.py:187-189), in one launch for up to 4 tokens (as
+    (engine/model.py:187-189), in one launch for up to 32 tokens (as
     :func:`rmsnorm_linear_group`)."""
     return _swiglu(x, gate, up, norm_weight, eps)
 

@@ -1,10 +1,10 @@
 """rms_norm fused into the projections that consume it (engine/model.py:166-170
 and :187-189): ``rmsnorm_linear_group`` and ``rmsnorm_swiglu``.
 
-Up to four tokens, K % 64 == 0 and a bf16 output run one launch whose
-skinny kernel normalises the activations it stages; every other case runs
-the RMSNorm kernel into the workspace and then the plain projection.  Both
-are checked:
+Up to four tokens (a group up to 32 of them where K fits the launch's
+registers), K % 64 == 0 and a bf16 output run one launch whose skinny kernel
+normalises the activations it loads; every other case runs the RMSNorm kernel
+into the workspace and then the plain projection.  Both are checked:
 
 - against the oracle chain ``linear(rmsnorm(x))`` within the linear
   tolerance (random inputs);
@@ -209,3 +209,44 @@ def test_fallback_leaves_the_pair_slots_empty(gpu):
     Q.rmsnorm_linear_group(x16, bf16_gpu(norm_weight(55, 2048), gpu), 1e-6, [wide])
     torch.cuda.synchronize()
     assert torch.equal(down.linear(x5), before)
+
+
+@pytest.mark.parametrize("m", [1, 4, 5, 8, 9, 16, 17, 31, 32, 33])
+@pytest.mark.parametrize("ns,k,hd", [([2048, 256, 256], 2048, 128), ([896, 128, 128], 896, 64), ([192, 96, 40], 640, 96),
+                                     ([512, 64, 64], 1024, 64), ([320, 160, 64], 512, 160), ([160, 80, 48], 512, 80)])
+def test_qkv_rope_equals_the_separate_calls(gpu, m, ns, k, hd):
+    """The norm, q|k|v and the rotation of q and k as one call, bit for bit
+    against rmsnorm, linear_group and rope_qk (inputs whose sum of squares is
+    exact, so that both norms agree): every staging of the tokens, head sizes
+    whose halves start on a block row (hd % 32 == 0) and one whose do not
+    (80: the separate rotation), folded plans, and 33 tokens (tiled GEMM)."""
+    _, qws, _ = group(gpu, 7 * k + hd, ns, k)
+    x = bf16_gpu(exact_sum_inputs(m * 5 + k + hd, m, k), gpu)
+    w = bf16_gpu(norm_weight(k + 2, k), gpu)
+    rng = np.random.default_rng(hd + m)
+    bs = [bf16_gpu(O.round_to_bf16(rng.standard_normal(n).astype(np.float32)), gpu) for n in ns]
+    cos, sin = (bf16_gpu(O.round_to_bf16(rng.standard_normal((m, hd)).astype(np.float32)), gpu) for _ in "cs")
+    q, kk, v = Q.linear_group(Q.rmsnorm(x, w, 1e-6), qws, bs)
+    q, kk = Q.rope_qk(q.view(m, -1, hd), kk.view(m, -1, hd), cos, sin)
+    a, b, c = Q._rmsnorm_qkv_rope(x, w, 1e-6, qws, bs, cos, sin, hd)
+    if (ns, hd) == ([2048, 256, 256], 128) and 3 <= m <= 32:
+        assert "ROPE = true" in _native.last_plan()  # one launch
+    assert torch.equal(a, q.reshape(m, -1)) and torch.equal(b, kk.reshape(m, -1)) and torch.equal(c, v)
+
+
+def test_qkv_rope_of_random_rows_matches_oracle(gpu):
+    """Random rows through the oracle's chain, with a zero row and a row of
+    large values, at the token counts of each staging."""
+    ns, k, hd, eps = [2048, 256, 256], 2048, 128, 1e-6
+    ws, qws, qs = group(gpu, 71, ns, k)
+    w = norm_weight(72, k)
+    for m in (3, 7, 13, 27):
+        x = activations(73 + m, m, k)
+        x[1] = 0.0
+        x[2] *= np.float32(100.0)
+        cos, sin = np.ones((m, hd), np.float32), np.zeros((m, hd), np.float32)  # (the identity rotation)
+        outs = Q._rmsnorm_qkv_rope(bf16_gpu(x, gpu), bf16_gpu(w, gpu), eps, qws, None, bf16_gpu(cos, gpu),
+                                   bf16_gpu(sin, gpu), hd)
+        h, dh = O.rmsnorm(x, w, eps), O.rmsnorm_dx(x, w, eps)
+        for o, (q, s) in zip(outs, qs):
+            report(to_np(o), O.linear(h, q, s), k, f"qkv_rope m={m}", acc=O.acc_bound(h, q, s, dx=dh))

@@ -95,3 +95,21 @@ def test_pair_tiles_plan(gpu):
         ref = O.swiglu(x, ws["gate"][1], ws["gate"][2], ws["up"][1], ws["up"][2])
         acc = O.swiglu_acc(x, ws["gate"][1], ws["gate"][2], ws["up"][1], ws["up"][2])
         report(to_np(act), ref, hidden, f"pair tiles m={m} n={inter} k={hidden}", acc=acc)
+
+
+@pytest.mark.parametrize("m,inter,hidden,tiled", [(17, 4112, 2048, True), (32, 8192, 1024, True), (31, 8208, 1088, True),
+                                                  (24, 12288, 64, True), (20, 4096, 512, False),
+                                                  (18, 12304, 128, False), (25, 5000, 896, True)])
+def test_pair_tiles_with_two_token_blocks(gpu, m, inter, hidden, tiled):
+    """17..32 tokens at the edges of the two- and three-tile plans (257, 512,
+    513 and 768 row tiles; 16 and 17 chunks) and just outside them, a last
+    workgroup with missing tiles and a last tile with missing rows."""
+    from pageserve_amd import _native
+
+    ws = _mlp_weights(gpu, 700 + m + inter, inter, hidden)
+    x = activations(750 + m, m, hidden)
+    act = Q.swiglu(bf16_gpu(x, gpu), ws["gate"][0], ws["up"][0])
+    assert ("launch_pair_tiles" in _native.last_plan()) == tiled
+    ref = O.swiglu(x, *ws["gate"][1:], *ws["up"][1:])
+    report(to_np(act), ref, hidden, f"pair tiles m={m} inter={inter} K={hidden}",
+           acc=O.swiglu_acc(x, *ws["gate"][1:], *ws["up"][1:]))
