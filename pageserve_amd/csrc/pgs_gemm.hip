@@ -656,8 +656,13 @@ __device__ __forceinline__ void dma16(__amdgpu_buffer_rsrc_t r, uint16_t* lds, i
   __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)lds, 16, voff, soff, 0, 0);
 }
 
-template <int BM, int BN, int NMAT, bool OUT_F32, int WLEAD, int S, int OCC>
-__global__ __launch_bounds__(kThreads, OCC) void gemm_dma_kernel(const uint16_t* __restrict__ x, GemmArgs ga) {
+// KG = 2: the workgroup is two groups of four waves on alternate K steps, each
+// with its own stages, and group 1 hands its accumulators to group 0 through
+// LDS at the end: two of the K splits of a few-tile shape in one workgroup,
+// without partial tiles in memory (down_proj [2048, 11008] at 2048 tokens: both
+// splits, no reduce launch).
+template <int BM, int BN, int NMAT, bool OUT_F32, int WLEAD, int S, int OCC, int KG>
+__global__ __launch_bounds__(kThreads * KG, OCC) void gemm_dma_kernel(const uint16_t* __restrict__ x, GemmArgs ga) {
   constexpr int TM = BM / 16, TN = BN / 64;
   constexpr int WSETS = WLEAD + 1;
   constexpr int UNROLL = lcm3(WSETS, S, 1);
@@ -669,31 +674,32 @@ __global__ __launch_bounds__(kThreads, OCC) void gemm_dma_kernel(const uint16_t*
   // which only WLEAD weight steps were issued)
   static_assert(BM % 32 == 0 && BN % 64 == 0 && XL >= 1 && S >= 2 && S <= 8 && WLEAD >= 1 && WLEAD >= S - 3,
                 "tile / pipeline");
-  __shared__ __attribute__((aligned(16))) uint16_t st0[XS];
-  __shared__ __attribute__((aligned(16))) uint16_t st1[XS];
-  __shared__ __attribute__((aligned(16))) uint16_t st2[S > 2 ? XS : 1];
-  __shared__ __attribute__((aligned(16))) uint16_t st3[S > 3 ? XS : 1];
-  __shared__ __attribute__((aligned(16))) uint16_t st4[S > 4 ? XS : 1];
-  __shared__ __attribute__((aligned(16))) uint16_t st5[S > 5 ? XS : 1];
-  __shared__ __attribute__((aligned(16))) uint16_t st6[S > 6 ? XS : 1];
-  __shared__ __attribute__((aligned(16))) uint16_t st7[S > 7 ? XS : 1];
+  __shared__ __attribute__((aligned(16))) uint16_t st0[KG * XS];
+  __shared__ __attribute__((aligned(16))) uint16_t st1[KG * XS];
+  __shared__ __attribute__((aligned(16))) uint16_t st2[S > 2 ? KG * XS : 1];
+  __shared__ __attribute__((aligned(16))) uint16_t st3[S > 3 ? KG * XS : 1];
+  __shared__ __attribute__((aligned(16))) uint16_t st4[S > 4 ? KG * XS : 1];
+  __shared__ __attribute__((aligned(16))) uint16_t st5[S > 5 ? KG * XS : 1];
+  __shared__ __attribute__((aligned(16))) uint16_t st6[S > 6 ? KG * XS : 1];
+  __shared__ __attribute__((aligned(16))) uint16_t st7[S > 7 ? KG * XS : 1];
+  const int kg = KG > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x / kThreads) : 0;
   auto stage = [&](auto I) -> uint16_t* {
     constexpr int i = decltype(I)::value;
-    if constexpr (i == 0) return st0;
-    else if constexpr (i == 1) return st1;
-    else if constexpr (i == 2) return st2;
-    else if constexpr (i == 3) return st3;
-    else if constexpr (i == 4) return st4;
-    else if constexpr (i == 5) return st5;
-    else if constexpr (i == 6) return st6;
-    else return st7;
+    if constexpr (i == 0) return st0 + kg * XS;
+    else if constexpr (i == 1) return st1 + kg * XS;
+    else if constexpr (i == 2) return st2 + kg * XS;
+    else if constexpr (i == 3) return st3 + kg * XS;
+    else if constexpr (i == 4) return st4 + kg * XS;
+    else if constexpr (i == 5) return st5 + kg * XS;
+    else if constexpr (i == 6) return st6 + kg * XS;
+    else return st7 + kg * XS;
   };
 
   const GroupArgs& a = ga.g;
   const int M = ga.M, K = ga.K;
   // (the wave index is wave-uniform; readfirstlane makes that visible, so the
   // DMA's LDS address -- it goes to M0 -- stays a scalar)
-  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int tid = threadIdx.x & (kThreads - 1), lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int tiles_n = ga.tiles / ga.tiles_m;
   int vn, mt_all;
   block_order(xcd_remap(blockIdx.x, ga.tiles * ga.splits), tiles_n * ga.splits, ga.tiles_m, vn, mt_all);
@@ -708,7 +714,10 @@ __global__ __launch_bounds__(kThreads, OCC) void gemm_dma_kernel(const uint16_t*
   const int kb = K / kBK;
   const int kt0 = static_cast<int>(static_cast<int64_t>(s) * kb / ga.splits);
   const int kt1 = static_cast<int>(static_cast<int64_t>(s + 1) * kb / ga.splits);
-  const int iters = kt1 - kt0, last = kt1 - 1;
+  // this group's K steps: kt0 + kg, kt0 + kg + KG, ... < kt1 (every group runs
+  // `iters` steps; past its last one it repeats that step's loads, without MFMAs)
+  const int range = kt1 - kt0, iters = (range + KG - 1) / KG, first = kt0 + kg;
+  const int last = range > kg ? first + (range - 1 - kg) / KG * KG : kt0;
 
   const int blk0 = n0 >> 4, blocks = (N + 15) >> 4;
   __amdgpu_buffer_rsrc_t wres[NMAT];
@@ -799,12 +808,12 @@ __global__ __launch_bounds__(kThreads, OCC) void gemm_dma_kernel(const uint16_t*
   // MFMAs of j on set i % WSETS and stage i % S, then the barrier.
   auto step = [&](auto I, int j) {
     constexpr int i = decltype(I)::value;
-    const int kt = kt0 + j;
-    wload(min(kt + WLEAD, last), wset[(i + WLEAD) % WSETS]);
-    dma(stage(std::integral_constant<int, (i + S - 1) % S>{}), min(kt + S - 1, last));
+    const int kt = first + j * KG;
+    wload(min(kt + WLEAD * KG, last), wset[(i + WLEAD) % WSETS]);
+    dma(stage(std::integral_constant<int, (i + S - 1) % S>{}), min(kt + (S - 1) * KG, last));
     __builtin_amdgcn_sched_barrier(0);
     __builtin_amdgcn_s_setprio(1);
-    compute(wset[i % WSETS], stage(std::integral_constant<int, i % S>{}));
+    if (KG == 1 || kt < kt1) compute(wset[i % WSETS], stage(std::integral_constant<int, i % S>{}));
     __builtin_amdgcn_s_setprio(0);
     step_barrier();
   };
@@ -812,10 +821,10 @@ __global__ __launch_bounds__(kThreads, OCC) void gemm_dma_kernel(const uint16_t*
   // costs the accumulators their registers: the compiler then spills them)
   {
     // prologue: stages 0 .. S-2, then weights 0 .. WLEAD-1; wait for stage 0
-    static_for([&](auto J) { dma(stage(J), min(kt0 + decltype(J)::value, last)); },
+    static_for([&](auto J) { dma(stage(J), min(first + decltype(J)::value * KG, last)); },
                std::make_integer_sequence<int, S - 1>{});
 #pragma unroll
-    for (int j = 0; j < WLEAD; ++j) wload(min(kt0 + j, last), wset[j]);
+    for (int j = 0; j < WLEAD; ++j) wload(min(first + j * KG, last), wset[j]);
     constexpr int kPro = (S - 2) * XL + WLEAD * WL;
     constexpr int kProWait = 0xF70 | (kPro & 15) | ((kPro >> 4) << 14);
     static_assert(kPro < 64, "vmcnt range");
@@ -827,6 +836,37 @@ __global__ __launch_bounds__(kThreads, OCC) void gemm_dma_kernel(const uint16_t*
     // the workgroup ends and its LDS is handed to the next one
     __builtin_amdgcn_s_waitcnt(0xF70);
   }
+  if constexpr (KG > 1) {
+    static_assert(KG == 2, "two K groups");
+    // group 1's accumulators in halves of the token tiles that fit a stage
+    constexpr int HT = TM / 2;
+    static_assert(4 * NMAT * TN * HT * 1024 <= KG * XS * 2, "half an accumulator tile fits a stage");
+    f32x4* red = reinterpret_cast<f32x4*>(st0);
+#pragma unroll
+    for (int hf = 0; hf < 2; ++hf) {
+      __syncthreads();  // (every DMA has landed; the stage is free)
+      if (kg == 1) {
+#pragma unroll
+        for (int mat = 0; mat < NMAT; ++mat)
+#pragma unroll
+          for (int nt = 0; nt < TN; ++nt)
+#pragma unroll
+            for (int mt = 0; mt < HT; ++mt)
+              red[(((wave * NMAT + mat) * TN + nt) * HT + mt) * 64 + lane] = acc[mat][nt][hf * HT + mt];
+      }
+      __syncthreads();
+      if (kg == 0) {
+#pragma unroll
+        for (int mat = 0; mat < NMAT; ++mat)
+#pragma unroll
+          for (int nt = 0; nt < TN; ++nt)
+#pragma unroll
+            for (int mt = 0; mt < HT; ++mt)
+              acc[mat][nt][hf * HT + mt] += red[(((wave * NMAT + mat) * TN + nt) * HT + mt) * 64 + lane];
+      }
+    }
+    if (kg != 0) return;
+  }
   if (ga.splits > 1) {
     store_partials<TN, TM, NMAT>(acc, ga, t, s, wave, lane);
     return;
@@ -837,7 +877,7 @@ __global__ __launch_bounds__(kThreads, OCC) void gemm_dma_kernel(const uint16_t*
 // Sums the split partial tiles in split order and runs the epilogue.  One
 // thread per accumulator slot (4 consecutive output rows of one token) over
 // all tiles; partial reads are coalesced 16-byte loads.  With the split
-// count known (SPL = 2, 4, 8; 0: read at run time) every partial load is in
+// count known (SPL = 2, 3, 4, 8; 0: read at run time) every partial load is in
 // flight before the first add (a runtime loop waits for each in turn), and
 // the epilogue operands are requested before them; the sum is the same
 // ((0 + p0) + p1) + ... either way.
@@ -898,6 +938,8 @@ int launch_reduce(const GemmArgs& ga, hipStream_t st) {
   const dim3 grid(static_cast<unsigned>((slots + kThreads - 1) / kThreads));
   if (ga.splits == 2)
     hipLaunchKernelGGL((gemm_reduce_kernel<BM, BN, NMAT, OUT_F32, 2>), grid, dim3(kThreads), 0, st, ga);
+  else if (ga.splits == 3)
+    hipLaunchKernelGGL((gemm_reduce_kernel<BM, BN, NMAT, OUT_F32, 3>), grid, dim3(kThreads), 0, st, ga);
   else if (ga.splits == 4)
     hipLaunchKernelGGL((gemm_reduce_kernel<BM, BN, NMAT, OUT_F32, 4>), grid, dim3(kThreads), 0, st, ga);
   else if (ga.splits == 8)
@@ -929,12 +971,13 @@ int launch_k64(const uint16_t* x, const GemmArgs& ga, hipStream_t st) {
   return launch_reduce<BM, BN, NMAT, OUT_F32>(ga, st);
 }
 
-template <int BM, int BN, int NMAT, bool OUT_F32, int WLEAD, int S, int OCC>
+template <int BM, int BN, int NMAT, bool OUT_F32, int WLEAD, int S, int OCC, int KG = 1>
 int launch_dma(const uint16_t* x, const GemmArgs& ga, hipStream_t st) {
   const int64_t grid = static_cast<int64_t>(ga.tiles) * ga.splits;
-  note_launch(__PRETTY_FUNCTION__, grid, ga.splits, ga.splits > 1 ? "gemm_reduce_kernel" : nullptr);
-  hipLaunchKernelGGL((gemm_dma_kernel<BM, BN, NMAT, OUT_F32, WLEAD, S, OCC>), dim3(static_cast<unsigned>(grid)),
-                     dim3(kThreads), 0, st, x, ga);
+  // (the K splits of the plan: KG of them in a workgroup)
+  note_launch(__PRETTY_FUNCTION__, grid, ga.splits * KG, ga.splits > 1 ? "gemm_reduce_kernel" : nullptr);
+  hipLaunchKernelGGL((gemm_dma_kernel<BM, BN, NMAT, OUT_F32, WLEAD, S, OCC, KG>), dim3(static_cast<unsigned>(grid)),
+                     dim3(kThreads * KG), 0, st, x, ga);
   int rc = check_launch("w8a16 gemm kernel");
   if (rc || ga.splits == 1) return rc;
   return launch_reduce<BM, BN, NMAT, OUT_F32>(ga, st);
@@ -1138,13 +1181,44 @@ int launch_plan(const uint16_t* x, const GemmArgs& ga, const GemmPlan& plan, hip
   }
   if constexpr (NMAT == 1) {
     // (lm_head at 256 tokens: 155-161 vs 174-184 us with register-staged activations)
-    if (plan.bm == 128 && plan.bn == kBN && ga.K % kBK == 0) return launch_dma<128, kBN, 1, OUT_F32, 2, 3, 2>(x, ga, st);
+    if (plan.bm == 128 && plan.bn == kBN && ga.K % kBK == 0)
+      return plan.kg == 2 ? launch_dma<128, kBN, 1, OUT_F32, 2, 3, 2, 2>(x, ga, st)
+                          : launch_dma<128, kBN, 1, OUT_F32, 2, 3, 2>(x, ga, st);
   }
   if (plan.bm == 128) return fail(PGS_ERR_INVALID_ARGUMENT, "w8a16 gemm: no 128-token tile kernel for this shape");
   return plan.bm == 32 ? launch_bm<32, NMAT, OUT_F32>(x, ga, st) : launch_bm<64, NMAT, OUT_F32>(x, ga, st);
 }
 
 }  // namespace
+
+// K splits of a long K in 128 x 128 tiles (1 from 512 tiles on) and whether two
+// of them share a workgroup (kg = 2: eight waves, one workgroup per CU, half the
+// partial tiles; kg = 1: four waves, two per CU, which spreads few or unevenly
+// many workgroups better).  The cheapest by a cost in steps of about a
+// microsecond: the K steps of a CU (a lone four-wave workgroup takes 0.6 per
+// step) and, where a tile has more than one workgroup, the reduce launch (2.5)
+// and the partials' bytes, written and read (6 to 7 TB/s).  Measured us, kg = 1
+// -> 2: down_proj [2048, 11008] at 2048 tokens (two splits) 103 -> 96, at 640
+// (eight -> six) 45 -> 38, at 896 (eight -> four) 60 -> 51; but 77 -> 89 at 1450
+// tokens, 192 tiles; [896, 4864] at 1501 tokens 30 -> 24, at 300 13.7 -> 14.5.
+struct LongSplit {
+  int splits, kg;
+};
+static LongSplit long_k_split(int64_t tiles, int kb) {
+  if (tiles >= 512) return {1, 1};
+  LongSplit best{};
+  double best_cost = 0;
+  for (int kg = 2; kg >= 1; --kg)
+    for (int sp = 2; sp <= 8; sp += 2) {
+      if (kg == 1 && sp == 6) continue;
+      const int64_t wgs = tiles * (sp / kg);
+      const double rounds = kg == 2 ? 1.03 * static_cast<double>((wgs + 255) / 256)
+                                    : wgs <= 256 ? 0.6 : std::max(1.0, static_cast<double>(wgs) / 512);
+      const double cost = rounds * ((kb + sp - 1) / sp) + (sp > kg ? 2.5 + wgs * (128 * 128 * 8) / (kg == 2 ? 6e6 : 7e6) : 0.0);
+      if (best.splits == 0 || cost < best_cost) best_cost = cost, best = {sp, kg};
+    }
+  return best;
+}
 
 GemmPlan plan_gemm(int m, int k, int nmat, const int32_t* n, int members, bool can_split) {
   GemmPlan p{};
@@ -1241,15 +1315,12 @@ GemmPlan plan_gemm(int m, int k, int nmat, const int32_t* n, int members, bool c
   // no faster or slower: q|k|v at 2048 tokens 32.5 vs 29.3 us)
   if (nmat == 1 && k % kBK == 0 && p.bn == kBN && m >= 256 && tiles_for(128) >= 2048) p.bm = 128;
   // a long K (down_proj) above 256 tokens: 128 x 128 tiles, split K (up to
-  // 8 ways) until 512 workgroups (down_proj [2048, 11008] at 384 tokens
-  // 33.6-34.1 vs 35.6-36.9 us with eight splits, at 768 52.4-54.1 vs
-  // 57.3-58.8, at 1280 69.8 vs 79.3 and at 1536 78.7 vs 87-90 with four, at
-  // 2048 94.5 vs 99-104 with two; at 512 and 1024 tokens within noise of the
-  // plans below, at 256 no faster)
-  // (without a workspace only where the split would stop at one anyway, 512
-  // tiles and more, so that a call plans alike with or without one)
-  const bool long128 = nmat == 1 && k % kBK == 0 && p.bn == kBN && kb > 64 && m > 256 &&
-                       (can_split || tiles_for(128) >= 512);
+  // 8 ways; at 256 tokens no faster than the plan below)
+  const bool long_k = nmat == 1 && k % kBK == 0 && p.bn == kBN && kb > 64 && m > 256;
+  const LongSplit ls = long_k ? long_k_split(tiles_for(128), kb) : LongSplit{1, 1};
+  // (without a workspace only where no partial tiles are needed, so that a
+  // call plans alike with or without one)
+  const bool long128 = long_k && (can_split || ls.splits == ls.kg);
   if (long128) p.bm = 128;
   // a single matrix with a short K and few 64-token tiles: 32-token tiles
   // give the CUs work without splitting K
@@ -1259,7 +1330,8 @@ GemmPlan plan_gemm(int m, int k, int nmat, const int32_t* n, int members, bool c
   p.tiles = p.tiles_m * p.tiles_n;
   p.splits = 1;
   if (long128) {
-    while (p.splits < 8 && static_cast<int64_t>(p.tiles) * p.splits < 512) p.splits *= 2;
+    p.kg = ls.kg;
+    p.splits = ls.splits / ls.kg;
     return p;
   }
   // fewer than 256 output tiles: split K until about four workgroups per CU,

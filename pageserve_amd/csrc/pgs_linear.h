@@ -69,7 +69,7 @@ struct SkinnyPlan {
 // Launch plan of the tile GEMM (m > 16).
 struct GemmPlan {
   int bm, bn;     // output tile (tokens x weight rows)
-  int kg;         // K groups of four waves per workgroup (K % 64 == 0 kernel)
+  int kg;         // K groups of four waves per workgroup (K % 64 == 0 kernels)
   int tiles_m, tiles_n, tiles;
   int splits;     // workgroups per output tile along K
   bool once;      // the one-shot tile (16 or 32 tokens, K <= 2048)

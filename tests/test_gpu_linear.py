@@ -507,3 +507,26 @@ def test_one_shot_32_token_plan(gpu):
     assert "launch_once" in plan and tm2 in plan and "NT = 4" in plan, plan
     for j in range(3):
         report(to_np(outs[j]), O.linear(x, qs[j], ss[j]), k, f"once qkv[{j}]", acc=O.acc_bound(x, qs[j], ss[j]))
+
+
+@pytest.mark.parametrize("m,n,k,splits,f32", [(1800, 2000, 4160, 2, False), (1793, 2048, 4224, 2, True),
+                                              (640, 2048, 4160, 6, False), (700, 896, 4864, 8, False),
+                                              (257, 2048, 4160, 8, True)])
+def test_two_k_splits_per_workgroup(gpu, m, n, k, splits, f32):
+    """Long K in 128 x 128 tiles with two of the K splits in a workgroup
+    (launch_dma<..., KG = 2>): alone (no partial tiles), and with two, three
+    and four workgroups per tile; even and odd step counts (a group without a
+    last step), ragged M and N, bias, residual and fp32 outputs."""
+    qw, q, s, x, b = _problem(gpu, 7900 + m + k, m, n, k, bias=True)
+    xt, bt = bf16_gpu(x, gpu), bf16_gpu(b, gpu)
+    odt = torch.float32 if f32 else torch.bfloat16
+    y = qw.linear(xt, bt, out_dtype=odt)
+    plan = _plan_kernel()
+    assert "KG = 2" in plan and "BM = 128" in plan and f"splits={splits}" in plan, plan
+    rows = np.concatenate([np.random.default_rng(m).choice(m, 24, replace=False), [0, 127, 128, m - 1]])
+    report(to_np(y)[rows], O.linear(x[rows], q, s, b), k, f"two splits m={m} n={n} k={k}",
+           acc=O.acc_bound(x[rows], q, s, b))
+    assert torch.equal(y, qw.linear(xt, bt, out_dtype=odt))
+    if not f32:
+        res = bf16_gpu(activations(7901, m, n), gpu)
+        assert torch.equal(qw.linear(xt, bt, residual=res), res + y)
