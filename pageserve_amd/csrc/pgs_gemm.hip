@@ -109,12 +109,31 @@ __device__ __forceinline__ Rows4<NMAT> rows4(const GroupArgs& a, int g, int N, i
   return e;
 }
 
+// Residuals of rows nb .. nb+3 of a token (single matrices), raw bf16 pairs.
+// One 8-byte load where N and the pointer allow (`vec`), and without a branch
+// on the position (a token or rows past the end read the last ones, unused), so
+// that a tile's residuals are all in flight before its first store: loaded where
+// they are added, each token tile waited for its own round trip (o_proj [2048,
+// 2048] at 1024 tokens, one workgroup per CU, spent 8 us in its epilogue).
+__device__ __forceinline__ bool vec_res(const uint16_t* res, int N) {
+  return (N & 3) == 0 && (reinterpret_cast<uintptr_t>(res) & 7) == 0;
+}
+__device__ __forceinline__ u32x2 residual4(const uint16_t* res, bool vec, int M, int N, int m, int nb) {
+  const int64_t row = static_cast<int64_t>(min(m, M - 1)) * N;
+  if (vec) return *reinterpret_cast<const u32x2*>(res + row + min(nb, N - 4));
+  uint32_t v[4];
+#pragma unroll
+  for (int r = 0; r < 4; ++r) v[r] = res[row + min(nb + r, N - 1)];
+  return u32x2{v[0] | (v[1] << 16), v[2] | (v[3] << 16)};
+}
+
 // Rows nb .. nb+3 of token m from their fp32 sums: scale and bias, or SwiGLU,
-// then the residual (single matrices) and one vector store when the four
-// outputs are in range and aligned (`yvec`), else element stores.
+// then the residual (single matrices; the linear output rounded first,
+// engine/model.py:184, 190) and one vector store when the four outputs are in
+// range and aligned (`yvec`), else element stores.
 template <int NMAT, bool OUT_F32>
-__device__ __forceinline__ void store_rows4(const GroupArgs& a, int g, int N, int m, int nb, const Rows4<NMAT>& e,
-                                            const f32x4& v0, const f32x4& v1, void* y, bool yvec) {
+__device__ __forceinline__ void store_rows4(int N, int m, int nb, const Rows4<NMAT>& e, const f32x4& v0,
+                                            const f32x4& v1, bool has_res, u32x2 rv, void* y, bool yvec) {
   float v[4];
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
@@ -124,10 +143,12 @@ __device__ __forceinline__ void store_rows4(const GroupArgs& a, int g, int N, in
       v[r] = v0[r] * e.s0[r] + e.bv[r];
   }
   const int64_t base = static_cast<int64_t>(m) * N + nb;
-  const uint16_t* res = (NMAT == 2) ? nullptr : pick(a.res, g);
-  if (NMAT == 1 && res) {
+  if (NMAT == 1 && has_res) {
 #pragma unroll
-    for (int r = 0; r < 4; ++r) v[r] = add_residual<OUT_F32>(v[r], res, base + min(r, N - 1 - nb));
+    for (int r = 0; r < 4; ++r) {
+      const float l = OUT_F32 ? v[r] : bf16_bits_to_f32(f32_to_bf16_bits(v[r]));
+      v[r] = l + bf16_bits_to_f32(static_cast<uint16_t>(rv[r >> 1] >> (16 * (r & 1))));
+    }
   }
   if (yvec && nb + 3 < N) {
     if constexpr (OUT_F32)
@@ -156,15 +177,22 @@ __device__ __forceinline__ void store_tile(const f32x4 (&acc)[NMAT][TN][TM], con
                                            int N, int m0, int n0, int wave, int lr, int lg) {
   void* y = (NMAT == 2) ? a.y[0] : pick(a.y, g);
   const bool yvec = vec_out<OUT_F32>(y, N);
+  const uint16_t* res = (NMAT == 2) ? nullptr : pick(a.res, g);
+  const bool rvec = vec_res(res, N);
 #pragma unroll
   for (int nt = 0; nt < TN; ++nt) {
     const int nb = n0 + wave * (BN / 4) + nt * 16 + 4 * lg;
     const Rows4<NMAT> e = rows4<NMAT>(a, g, N, nb);
+    u32x2 rv[TM];
+    if (NMAT == 1 && res) {
+#pragma unroll
+      for (int mt = 0; mt < TM; ++mt) rv[mt] = residual4(res, rvec, M, N, m0 + mt * 16 + lr, nb);
+    }
 #pragma unroll
     for (int mt = 0; mt < TM; ++mt) {
       const int m = m0 + mt * 16 + lr;
       if (m >= M) continue;
-      store_rows4<NMAT, OUT_F32>(a, g, N, m, nb, e, acc[0][nt][mt], acc[NMAT - 1][nt][mt], y, yvec);
+      store_rows4<NMAT, OUT_F32>(N, m, nb, e, acc[0][nt][mt], acc[NMAT - 1][nt][mt], res != nullptr, rv[mt], y, yvec);
     }
   }
 }
@@ -874,6 +902,275 @@ __global__ __launch_bounds__(kThreads * KG, OCC) void gemm_dma_kernel(const uint
   store_tile<BN, TN, TM, NMAT, OUT_F32>(acc, a, g, M, N, m0, n0, wave, lr, lg);
 }
 
+// The tile on 32x32x16 MFMAs with the loop pipelined across its K steps, for
+// the shapes whose time is each wave's own chain of loads, LDS reads, widening
+// and MFMAs rather than one unit's throughput: few workgroups per CU.
+//  * v_mfma_f32_32x32x16_bf16 hides other instructions better than the 16x16x32
+//    form: 24 VALU and 8 LDS reads per 8 of them still run at 1718 TFLOP/s,
+//    against 1186 for 16 of the smaller (register operands, two waves per SIMD).
+//    The packed weights serve it unchanged: a 32-row operand is two 16-row
+//    blocks (lane l: row l % 16 of block (l / 16) % 2), a load covers the
+//    16-column groups i and 2 + i of the two lane halves, and a 16-row gate and
+//    up block pair becomes one operand by exchanging every second 16-lane row
+//    of the two loads (v_permlane16_swap).
+//  * A 64-wide K step is four sub-steps of 16 k.  While sub-step c's MFMAs run,
+//    the B fragments of c + 1 are read, its weights are widened and a share of
+//    the step's loads is issued between the MFMAs, the first sub-step of the
+//    next step included: the step's barrier stands before the last sub-step.
+//  * S stages of activations by LDS DMA; a stage is waited for one whole step
+//    before its first read (a read right behind the wait and the barrier has
+//    returned stale data here with stages written by other waves' DMAs).
+//  * KG = 2: two groups of NW waves on alternate K steps, as in gemm_dma_kernel.
+//  * The epilogue's scales, bias and residuals are loaded before the loop.
+// Wave (wn, wm) of a group owns BN / (NW / WM) rows of each matrix and BM / WM
+// tokens.  No K split across workgroups.
+__device__ __forceinline__ f32x16 mfma32x32x16(bf16x8 a, bf16x8 b, f32x16 c) {
+  return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
+}
+
+template <int BM, int BN, int NMAT, bool OUT_F32, int KG, int NW, int WM, int WLEAD, int S, int OCC>
+__global__ __launch_bounds__(64 * NW * KG, OCC) void gemm_pipe_kernel(const uint16_t* __restrict__ x, GemmArgs ga) {
+  constexpr int WN = NW / WM;           // waves along the weight rows
+  constexpr int RPM = BN / WN;          // rows per matrix and wave
+  constexpr bool SWAP = NMAT == 2;      // 16 gate and 16 up rows in one operand
+  constexpr int TB = BM / WM / 32;      // 32-token tiles per wave
+  static_assert(NW == WN * WM && RPM == (SWAP ? 16 : 32) && TB * WM * 32 == BM, "one 32-row operand per wave");
+  constexpr int WSETS = WLEAD + 1;
+  constexpr int UNROLL = lcm3(WSETS, S, 1);
+  constexpr int XS = BM * kBK;              // bf16 elements of one stage
+  constexpr int XL = BM * 8 / (64 * NW);    // DMA instructions per lane per stage
+  constexpr int WL = 2;                     // weight loads per lane per step
+  constexpr int OPS = WL + XL, SLOTS = 4 * TB;
+  static_assert(XL * 64 * NW == BM * 8 && S >= 4 && S <= 5 && WLEAD >= 1 && OPS <= SLOTS, "pipeline");
+  __shared__ __attribute__((aligned(16))) uint16_t st0[KG * XS];
+  __shared__ __attribute__((aligned(16))) uint16_t st1[KG * XS];
+  __shared__ __attribute__((aligned(16))) uint16_t st2[KG * XS];
+  __shared__ __attribute__((aligned(16))) uint16_t st3[KG * XS];
+  __shared__ __attribute__((aligned(16))) uint16_t st4[S > 4 ? KG * XS : 1];
+  const int kg = KG > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x / (64 * NW)) : 0;
+  auto stage = [&](auto I) -> uint16_t* {
+    constexpr int i = decltype(I)::value;
+    if constexpr (i == 0) return st0 + kg * XS;
+    else if constexpr (i == 1) return st1 + kg * XS;
+    else if constexpr (i == 2) return st2 + kg * XS;
+    else if constexpr (i == 3) return st3 + kg * XS;
+    else return st4 + kg * XS;
+  };
+
+  const GroupArgs& a = ga.g;
+  const int M = ga.M, K = ga.K;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((threadIdx.x >> 6) % NW);
+  const int wn = wave / WM, wm = wave % WM;
+  const int tiles_n = ga.tiles / ga.tiles_m;
+  int nt_all, mt_all;
+  block_order(xcd_remap(blockIdx.x, ga.tiles), tiles_n, ga.tiles_m, nt_all, mt_all);
+  int g = 0;
+#pragma unroll
+  for (int i = 1; i < PGS_MAX_GROUP; ++i) g = (NMAT == 1 && i < a.n_outs && nt_all >= a.unit_begin[i]) ? i : g;
+  const int N = pick(a.n, g);
+  const int n0 = (nt_all - pick(a.unit_begin, g)) * BN;
+  const int m0 = mt_all * BM;
+  const int kb = K / kBK;
+  // this group's K steps: kg, kg + KG, ... < kb (every group runs `iters`
+  // steps; past its last one it repeats that step's loads, without MFMAs)
+  const int iters = (kb + KG - 1) / KG;
+  const int last = kb > kg ? kg + (kb - 1 - kg) / KG * KG : 0;
+
+  const int blk0 = n0 >> 4, blocks = (N + 15) >> 4;
+  __amdgpu_buffer_rsrc_t wres[NMAT];
+#pragma unroll
+  for (int mat = 0; mat < NMAT; ++mat) {
+    const int8_t* qg = (NMAT == 2) ? a.q[mat] : pick(a.q, g);
+    wres[mat] = make_rsrc(qg + static_cast<int64_t>(blk0) * kb * 1024, static_cast<int64_t>(blocks - blk0) * kb * 1024);
+  }
+  const int h = lane >> 5;
+  const int woff = SWAP ? wn * kb * 1024 + lane * 16
+                        : (wn * 2 + ((lane >> 4) & 1)) * kb * 1024 + ((lane & 15) + 32 * h) * 16;
+  // activations: rows m0.. of x; rows past M read as zero.  DMA j of this wave
+  // fills positions as in gemm_dma_kernel
+  const __amdgpu_buffer_rsrc_t xres = make_rsrc(x + static_cast<int64_t>(m0) * K, static_cast<int64_t>(M - m0) * K * 2);
+  int xoff_g[XL];
+#pragma unroll
+  for (int j = 0; j < XL; ++j) {
+    const int p = (wave * XL + j) * 64 + lane;
+    const int row = p >> 3;
+    const int ch = (p & 7) ^ (row & 7) ^ ((row >> 3) & 1);
+    xoff_g[j] = row * K * 2 + ch * 16;
+  }
+  // B operand of sub-step c: 16-byte chunk 4 h + c of token lane % 32 (the
+  // weights' k order: lane half h holds columns 32 h .. 32 h + 31)
+  int bofs[4];
+#pragma unroll
+  for (int c = 0; c < 4; ++c) bofs[c] = wm * (BM / WM) * kBK + swz(lane & 31, 4 * h + c);
+
+  using WRegs = u32x4[2];
+  WRegs wset[WSETS];
+  auto wload1 = [&](int o, int kt, WRegs& w) {
+    w[o] = SWAP ? __builtin_amdgcn_raw_buffer_load_b128(wres[o % NMAT], woff, kt * 1024, 0)
+                : __builtin_amdgcn_raw_buffer_load_b128(wres[0], woff + o * 256, kt * 1024, 0);
+  };
+  auto dma1 = [&](uint16_t* dst, int j, int kt) {
+    dma16(xres, dst + (wave * XL + j) * 512, xoff_g[j], kt * (kBK * 2));
+  };
+  // quad q of a 32x32 tile holds rows 8 q + 4 h .. + 3 of token lane % 32; of
+  // the pair, quads 0 and 1 are gate rows, 2 and 3 the same up rows
+  constexpr int QUADS = SWAP ? 2 : 4;
+  Rows4<NMAT> epi[QUADS];
+#pragma unroll
+  for (int q = 0; q < QUADS; ++q) epi[q] = rows4<NMAT>(a, g, N, n0 + wn * RPM + 8 * q + 4 * h);
+  const uint16_t* res = (NMAT == 2) ? nullptr : pick(a.res, g);
+  u32x2 rv[QUADS][TB];
+  if (NMAT == 1 && res) {
+    const bool rvec = vec_res(res, N);
+#pragma unroll
+    for (int q = 0; q < QUADS; ++q)
+#pragma unroll
+      for (int j = 0; j < TB; ++j)
+        rv[q][j] = residual4(res, rvec, M, N, m0 + wm * (BM / WM) + j * 32 + (lane & 31), n0 + wn * RPM + 8 * q + 4 * h);
+  }
+  f32x16 acc[TB];
+#pragma unroll
+  for (int j = 0; j < TB; ++j)
+#pragma unroll
+    for (int e = 0; e < 16; ++e) acc[j][e] = 0.f;
+
+  bf16x8 bx[2][TB], aw[2];
+  auto rd = [&](int c, const uint16_t* stg) {
+#pragma unroll
+    for (int j = 0; j < TB; ++j) bx[c & 1][j] = *reinterpret_cast<const bf16x8*>(stg + bofs[c] + j * 32 * kBK);
+  };
+  auto widen = [&](int c, const WRegs& w) {
+    aw[c & 1] = i8x8_to_bf16x8(w[c >> 1][2 * (c & 1)], w[c >> 1][2 * (c & 1) + 1]);
+  };
+  auto pair_operand = [&](WRegs& w) {
+    if constexpr (SWAP) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const auto r = __builtin_amdgcn_permlane16_swap(w[0][e], w[1][e], false, false);
+        w[0][e] = r[0];
+        w[1][e] = r[1];
+      }
+    }
+  };
+  // A step issues its weight loads, then its DMAs, spread over the MFMAs: load
+  // o behind MFMA o * SLOTS / OPS.  At its barrier, behind the third sub-step,
+  // each wave has waited for its own DMAs of the stage two steps on (issued
+  // S - 3 steps ago; n012 of this step's loads are younger, and all of each
+  // step between).
+  constexpr int n012 = (3 * TB * OPS + SLOTS - 1) / SLOTS;
+  constexpr int kAfter = (S - 4) * OPS + n012;
+  constexpr int kWait = 0xF70 | (kAfter & 15) | ((kAfter >> 4) << 14);
+  static_assert(kAfter < 64, "vmcnt range");
+  auto step = [&](auto I, int j) {
+    constexpr int i = decltype(I)::value;
+    const int kt = kg + j * KG;
+    const int ktw = min(kt + WLEAD * KG, last), ktx = min(kt + (S - 1) * KG, last);
+    const bool on = KG == 1 || kt < kb;
+    uint16_t* const cur = stage(std::integral_constant<int, i % S>{});
+    uint16_t* const nxt = stage(std::integral_constant<int, (i + 1) % S>{});
+    uint16_t* const fill = stage(std::integral_constant<int, (i + S - 1) % S>{});
+    WRegs& wl = wset[(i + WLEAD) % WSETS];
+    WRegs& wc = wset[i % WSETS];
+    WRegs& wnext = wset[(i + 1) % WSETS];
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      if (c < 3) rd(c + 1, cur);
+      else rd(0, nxt);
+      if (c == 3) pair_operand(wnext);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int jj = 0; jj < TB; ++jj) {
+        if (on) acc[jj] = mfma32x32x16(aw[c & 1], bx[c & 1][jj], acc[jj]);
+        if (jj == 0) {
+          if (c < 3) widen(c + 1, wc);
+          else widen(0, wnext);
+        }
+#pragma unroll
+        for (int o = 0; o < OPS; ++o)
+          if (o * SLOTS / OPS == c * TB + jj) {
+            if (o < WL) wload1(o, ktw, wl);
+            else dma1(fill, o - WL, ktx);
+          }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      if (c == 2) {
+        __builtin_amdgcn_s_waitcnt(kWait);
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+      }
+    }
+  };
+  {
+    // prologue: stages 0 .. S-2, then weights 0 .. WLEAD-1 (in this order: the
+    // count below relies on it); stages 0 and 1 have landed at the barrier, and
+    // stage 0 is read behind the arrival of the first weights, issued last
+    static_for([&](auto J) {
+#pragma unroll
+      for (int j = 0; j < XL; ++j) dma1(stage(J), j, min(kg + decltype(J)::value * KG, last));
+    }, std::make_integer_sequence<int, S - 1>{});
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int j = 0; j < WLEAD; ++j)
+#pragma unroll
+      for (int o = 0; o < WL; ++o) wload1(o, min(kg + j * KG, last), wset[j]);
+    __builtin_amdgcn_sched_barrier(0);
+    constexpr int kPro = (S - 3) * XL + WLEAD * WL;
+    constexpr int kProWait = 0xF70 | (kPro & 15) | ((kPro >> 4) << 14);
+    static_assert(kPro < 64, "vmcnt range");
+    __builtin_amdgcn_s_waitcnt(kProWait);
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    pair_operand(wset[0]);
+    widen(0, wset[0]);
+    __builtin_amdgcn_sched_barrier(0);
+    rd(0, stage(std::integral_constant<int, 0>{}));
+    run_blocks(step, iters, std::make_integer_sequence<int, UNROLL>{});
+    // the last steps' repeated loads land before the LDS is used again or
+    // handed to the next workgroup
+    __builtin_amdgcn_s_waitcnt(0xF70);
+  }
+  if constexpr (KG > 1) {
+    static_assert(KG == 2 && NW * 4 * 64 * 16 <= KG * XS * 2, "a token tile of every wave fits a stage");
+    f32x4* red = reinterpret_cast<f32x4*>(st0);
+#pragma unroll
+    for (int j = 0; j < TB; ++j) {
+      __syncthreads();
+      if (kg == 1) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+          red[(wave * 4 + q) * 64 + lane] = f32x4{acc[j][4 * q], acc[j][4 * q + 1], acc[j][4 * q + 2], acc[j][4 * q + 3]};
+      }
+      __syncthreads();
+      if (kg == 0) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const f32x4 v = red[(wave * 4 + q) * 64 + lane];
+#pragma unroll
+          for (int r = 0; r < 4; ++r) acc[j][4 * q + r] += v[r];
+        }
+      }
+    }
+    if (kg != 0) return;
+  }
+  void* y = (NMAT == 2) ? a.y[0] : pick(a.y, g);
+  const bool yvec = vec_out<OUT_F32>(y, N);
+#pragma unroll
+  for (int q = 0; q < QUADS; ++q)
+#pragma unroll
+    for (int j = 0; j < TB; ++j) {
+      const int m = m0 + wm * (BM / WM) + j * 32 + (lane & 31);
+      f32x4 v0, v1;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        v0[r] = acc[j][4 * q + r];
+        v1[r] = acc[j][(SWAP ? 8 : 0) + 4 * q + r];
+      }
+      if (m < M)
+        store_rows4<NMAT, OUT_F32>(N, m, n0 + wn * RPM + 8 * q + 4 * h, epi[q], v0, v1, res != nullptr, rv[q][j], y, yvec);
+    }
+}
+
 // Sums the split partial tiles in split order and runs the epilogue.  One
 // thread per accumulator slot (4 consecutive output rows of one token) over
 // all tiles; partial reads are coalesced 16-byte loads.  With the split
@@ -907,6 +1204,9 @@ __global__ __launch_bounds__(kThreads) void gemm_reduce_kernel(GemmArgs ga) {
   const int nb = n0 + wave * (BN / 4) + nt * 16 + 4 * (lane >> 4);
   if (m >= M) return;
   const Rows4<NMAT> e = rows4<NMAT>(a, g, N, nb);
+  const uint16_t* res = (NMAT == 2) ? nullptr : pick(a.res, g);
+  u32x2 rv = {0u, 0u};
+  if (NMAT == 1 && res) rv = residual4(res, vec_res(res, N), M, N, m, nb);
   const f32x4* part = reinterpret_cast<const f32x4*>(ga.partials) + static_cast<int64_t>(t) * ga.splits * NMAT * SLOTS;
   f32x4 v[NMAT];
   if constexpr (SPL > 0) {
@@ -929,7 +1229,7 @@ __global__ __launch_bounds__(kThreads) void gemm_reduce_kernel(GemmArgs ga) {
     }
   }
   void* y = (NMAT == 2) ? a.y[0] : pick(a.y, g);
-  store_rows4<NMAT, OUT_F32>(a, g, N, m, nb, e, v[0], v[NMAT - 1], y, vec_out<OUT_F32>(y, N));
+  store_rows4<NMAT, OUT_F32>(N, m, nb, e, v[0], v[NMAT - 1], res != nullptr, rv, y, vec_out<OUT_F32>(y, N));
 }
 
 template <int BM, int BN, int NMAT, bool OUT_F32>
@@ -981,6 +1281,16 @@ int launch_dma(const uint16_t* x, const GemmArgs& ga, hipStream_t st) {
   int rc = check_launch("w8a16 gemm kernel");
   if (rc || ga.splits == 1) return rc;
   return launch_reduce<BM, BN, NMAT, OUT_F32>(ga, st);
+}
+
+template <int BM, int BN, int NMAT, bool OUT_F32, int KG, int NW, int WM, int WLEAD, int S, int OCC>
+int launch_pipe(const uint16_t* x, const GemmArgs& ga, hipStream_t st) {
+  if (ga.splits != 1 || ga.K % kBK != 0)
+    return fail(PGS_ERR_INVALID_ARGUMENT, "w8a16 gemm: pipelined tile for K=%d, %d splits", ga.K, ga.splits);
+  note_launch(__PRETTY_FUNCTION__, ga.tiles, 1);
+  hipLaunchKernelGGL((gemm_pipe_kernel<BM, BN, NMAT, OUT_F32, KG, NW, WM, WLEAD, S, OCC>),
+                     dim3(static_cast<unsigned>(ga.tiles)), dim3(64 * NW * KG), 0, st, x, ga);
+  return check_launch("w8a16 gemm kernel");
 }
 
 // A short K over few tokens in one round trip (single matrices at 33..128
@@ -1046,6 +1356,14 @@ __global__ __launch_bounds__(1024) void gemm_once_kernel(const uint16_t* __restr
   const int lr = lane & 15, lg = lane >> 4;
   const int nb = n0 + nt * 16 + 4 * lg;
   const Rows4<1> e = rows4<1>(a, g, N, nb);
+  const uint16_t* res = pick(a.res, g);
+  u32x2 rv[TM];
+  if (res) {
+#pragma unroll
+    for (int t = 0; t < TM; ++t) rv[t] = residual4(res, vec_res(res, N), M, N, m0 + 16 * t + lr, nb);
+  }
+  // (the count below expects the weight loads to be the youngest)
+  __builtin_amdgcn_sched_barrier(0);
   // weights, last: this wave's tile, chunks grp, grp + NG, ... (CPG of
   // them; a chunk past K is never used)
   const int blk0 = n0 >> 4, blocks = (N + 15) >> 4;
@@ -1100,7 +1418,7 @@ __global__ __launch_bounds__(1024) void gemm_once_kernel(const uint16_t* __restr
 #pragma unroll
     for (int q = 1; q < NG; ++q) v += red[((q * NT + nt) * TM + t) * 64 + lane];
     const int m = m0 + 16 * t + lr;
-    if (m < M) store_rows4<1, OUT_F32>(a, g, N, m, nb, e, v, v, y, vec_out<OUT_F32>(y, N));
+    if (m < M) store_rows4<1, OUT_F32>(N, m, nb, e, v, v, res != nullptr, rv[t], y, vec_out<OUT_F32>(y, N));
   }
 }
 
@@ -1114,26 +1432,26 @@ int launch_once(const uint16_t* x, const GemmArgs& ga, hipStream_t st) {
   return check_launch("w8a16 gemm kernel");
 }
 
-// Measured on MI355X (Qwen2.5-3B projections, 512, 1024 and 2048 tokens).
-// K % 64 == 0: at least two work units per CU without a K split (q|k|v, o
-// and down_proj at 2048 tokens): the LDS-DMA kernel, 4 waves per SIMD
-// (o 23.4 vs 24.6 us, q|k|v 29.5 vs 30.5 us at 2048 tokens); at most two
-// work units per CU (o / q|k|v / down_proj at 512 and 1024 tokens): the
-// buffer-load kernel in two K groups per workgroup, or, for a long K over
-// at most one work unit per CU (measured on down_proj at 1024 tokens, which
-// now takes the 128 x 128 split plan, as fast there), four.  Other K:
-// the pointer kernel (SwiGLU: one-step pipeline at the compiler's register
-// budget; single matrices: two-step pipeline at 4 waves per SIMD).
+// The tiles of 128 rows that no plan above takes.  K % 64 == 0 (single matrices
+// in 64-token tiles): many units without a K split, 512 and more: the LDS-DMA
+// kernel, 4 waves per SIMD (q|k|v at 2048 tokens 29.5 vs 30.5 us); a long K over
+// at most one work unit per CU (few tiles at up to 256 tokens): four K groups of
+// the buffer-load kernel, else two.  Other K: the pointer kernel (SwiGLU:
+// one-step pipeline at the compiler's register budget; single matrices: two-step
+// pipeline at 4 waves per SIMD).
 template <int BM, int NMAT, bool OUT_F32>
 int launch_bm(const uint16_t* x, const GemmArgs& ga, hipStream_t st) {
-  if (ga.K % kBK == 0) {
-    if constexpr (NMAT == 2) return launch_k64<BM, kBN, 2, OUT_F32, 2, 2, 2>(x, ga, st);
-    const int64_t units = static_cast<int64_t>(ga.tiles) * ga.splits;
-    // a long K over at most one workgroup per CU: four K groups
-    if (units <= 256 && ga.K / kBK > 64) return launch_k64<BM, kBN, 1, OUT_F32, 2, 2, 1, 4>(x, ga, st);
-    if (units >= 512 && ga.splits == 1) return launch_dma<BM, kBN, 1, OUT_F32, 2, 3, 4>(x, ga, st);
-    return launch_k64<BM, kBN, 1, OUT_F32, 2, 2, 2, 2>(x, ga, st);
+  if constexpr (NMAT == 1 && BM == 64) {
+    if (ga.K % kBK == 0) {
+      const int64_t units = static_cast<int64_t>(ga.tiles) * ga.splits;
+      // a long K over at most one workgroup per CU: four K groups
+      if (units <= 256 && ga.K / kBK > 64) return launch_k64<BM, kBN, 1, OUT_F32, 2, 2, 1, 4>(x, ga, st);
+      if (units >= 512 && ga.splits == 1) return launch_dma<BM, kBN, 1, OUT_F32, 2, 3, 4>(x, ga, st);
+      return launch_k64<BM, kBN, 1, OUT_F32, 2, 2, 2, 2>(x, ga, st);
+    }
   }
+  if (ga.K % kBK == 0)
+    return fail(PGS_ERR_INVALID_ARGUMENT, "w8a16 gemm: no %d-token tile kernel for K=%d", BM, ga.K);
   if constexpr (NMAT == 2)
     return launch_cfg<BM, kBN, 2, OUT_F32, 1, 1>(x, ga, st);
   else
@@ -1142,6 +1460,16 @@ int launch_bm(const uint16_t* x, const GemmArgs& ga, hipStream_t st) {
 
 template <int NMAT, bool OUT_F32>
 int launch_plan(const uint16_t* x, const GemmArgs& ga, const GemmPlan& plan, hipStream_t st) {
+  if (plan.pipe) {
+    if constexpr (NMAT == 2) {
+      if (plan.bm == 64) return launch_pipe<64, 64, 2, OUT_F32, 1, 4, 1, 4, 5, 2>(x, ga, st);
+      if (plan.bm == 96) return launch_pipe<96, 64, 2, OUT_F32, 1, 4, 1, 4, 5, 1>(x, ga, st);
+      return launch_pipe<128, 64, 2, OUT_F32, 1, 8, 2, 4, 5, 2>(x, ga, st);
+    } else {
+      return plan.kg == 2 ? launch_pipe<64, 128, 1, OUT_F32, 2, 4, 1, 2, 4, 1>(x, ga, st)
+                          : launch_pipe<64, 128, 1, OUT_F32, 1, 4, 1, 2, 4, 2>(x, ga, st);
+    }
+  }
   if constexpr (NMAT == 1) {
     // one-shot 16- or 32-token tiles (K <= 2048): 64, 32 or 16 rows in 4, 8
     // or 16 K groups
@@ -1195,27 +1523,28 @@ int launch_plan(const uint16_t* x, const GemmArgs& ga, const GemmPlan& plan, hip
 // of them share a workgroup (kg = 2: eight waves, one workgroup per CU, half the
 // partial tiles; kg = 1: four waves, two per CU, which spreads few or unevenly
 // many workgroups better).  The cheapest by a cost in steps of about a
-// microsecond: the K steps of a CU (a lone four-wave workgroup takes 0.6 per
+// microsecond: the K steps of a CU (a lone four-wave workgroup takes 0.7 per
 // step) and, where a tile has more than one workgroup, the reduce launch (2.5)
-// and the partials' bytes, written and read (6 to 7 TB/s).  Measured us, kg = 1
-// -> 2: down_proj [2048, 11008] at 2048 tokens (two splits) 103 -> 96, at 640
-// (eight -> six) 45 -> 38, at 896 (eight -> four) 60 -> 51; but 77 -> 89 at 1450
-// tokens, 192 tiles; [896, 4864] at 1501 tokens 30 -> 24, at 300 13.7 -> 14.5.
+// and the partials' bytes, written and read (5 and 6.5 TB/s).  Measured in a
+// layer, GEMM + reduce us, kg = 1 -> 2: down_proj [2048, 11008] at 2048 tokens
+// (two splits) 104 -> 99, at 640 (eight -> six) 49 -> 42, at 512 (eight) 37 ->
+// 35; but at 1024 (four) 58 -> 60 and at 1450, 192 tiles, 12 us more.
 struct LongSplit {
   int splits, kg;
+  double cost;
 };
 static LongSplit long_k_split(int64_t tiles, int kb) {
-  if (tiles >= 512) return {1, 1};
+  if (tiles >= 512) return {1, 1, 0.0};
   LongSplit best{};
   double best_cost = 0;
   for (int kg = 2; kg >= 1; --kg)
     for (int sp = 2; sp <= 8; sp += 2) {
       if (kg == 1 && sp == 6) continue;
       const int64_t wgs = tiles * (sp / kg);
-      const double rounds = kg == 2 ? 1.03 * static_cast<double>((wgs + 255) / 256)
-                                    : wgs <= 256 ? 0.6 : std::max(1.0, static_cast<double>(wgs) / 512);
-      const double cost = rounds * ((kb + sp - 1) / sp) + (sp > kg ? 2.5 + wgs * (128 * 128 * 8) / (kg == 2 ? 6e6 : 7e6) : 0.0);
-      if (best.splits == 0 || cost < best_cost) best_cost = cost, best = {sp, kg};
+      const double rounds = kg == 2 ? 1.1 * static_cast<double>((wgs + 255) / 256)
+                                    : wgs <= 256 ? 0.7 : std::max(1.0, static_cast<double>(wgs) / 512);
+      const double cost = rounds * ((kb + sp - 1) / sp) + (sp > kg ? 2.5 + wgs * (128 * 128 * 8) / (kg == 2 ? 5e6 : 6.5e6) : 0.0);
+      if (best.splits == 0 || cost < best_cost) best_cost = cost, best = {sp, kg, cost};
     }
   return best;
 }
@@ -1286,6 +1615,22 @@ GemmPlan plan_gemm(int m, int k, int nmat, const int32_t* n, int members, bool c
         return p;
       }
     }
+    // the SwiGLU pair above 64 tokens where one round of pipelined tiles covers
+    // it: 64 tokens if those tiles number at most 256, else one token tile of 96
+    // or 128 (11008 x 2048 at 66 / 100 / 128 tokens 21.7 / 23.0 / 23.4 -> 16.3 /
+    // 19.5 / 20.2 us, 4864 x 896 at 100 11.9 -> 7.9 us)
+    if (nmat == 2 && m > 64) {
+      const int bm = tiles_for(64) <= 256 ? 64 : m <= 96 ? 96 : 128;
+      if (tiles_for(bm) <= 256) {
+        p.pipe = true;
+        p.bm = bm;
+        p.tiles_m = (m + bm - 1) / bm;
+        p.tiles_n = tiles_n;
+        p.tiles = p.tiles_m * tiles_n;
+        p.splits = 1;
+        return p;
+      }
+    }
     p.bm = (nmat == 1 && kb <= 64) ? 32 : 64;
     // the SwiGLU pair above 96 tokens: one 128-token tile row, each weight
     // panel read once (128 tokens 21.9 vs 23.5 us; at 96 tokens within noise)
@@ -1317,10 +1662,38 @@ GemmPlan plan_gemm(int m, int k, int nmat, const int32_t* n, int members, bool c
   // a long K (down_proj) above 256 tokens: 128 x 128 tiles, split K (up to
   // 8 ways; at 256 tokens no faster than the plan below)
   const bool long_k = nmat == 1 && k % kBK == 0 && p.bn == kBN && kb > 64 && m > 256;
-  const LongSplit ls = long_k ? long_k_split(tiles_for(128), kb) : LongSplit{1, 1};
+  const LongSplit ls = long_k ? long_k_split(tiles_for(128), kb) : LongSplit{1, 1, 0.0};
   // (without a workspace only where no partial tiles are needed, so that a
   // call plans alike with or without one)
   const bool long128 = long_k && (can_split || ls.splits == ls.kg);
+  // pipelined 64 x 128 tiles without a K split, one round of them: two K groups
+  // (one workgroup per CU) for at most 256 tiles of a longer K, one group (two
+  // per CU) for up to 512.  Short K: q|k|v [2560, 2048] at 640 / 768 / 1024 /
+  // 1280 tokens 16.9 / 17.2 / 21.8 / 23.4 -> 14.2 / 15.7 / 19.8 / 21.3 us, o_proj
+  // [2048, 2048] at 896 / 1024 / 1501 / 2048 16.9 / 16.3 / 22.6 / 24.5 -> 14.5 /
+  // 14.8 / 20.7 / 23.7, [1152, 896] at 1501 11.0 -> 9.7; more tiles are slower
+  // (560: 28.9 vs 30.0).  Long K of up to 96 steps: where its steps cost less
+  // than the split above, in the same measure ([896, 4864] at 1280 / 1501 / 2048
+  // tokens 27.3 / 29.8 / 36.7 before either -> 22.8 / 23.4 / 25.7).
+  if (nmat == 1 && k % kBK == 0 && p.bn == kBN && m > 128) {
+    const int64_t t64 = tiles_for(64);
+    int kg = 0;
+    if (kb <= 64)
+      kg = t64 > 512 ? 0 : kb >= 32 && t64 <= 256 ? 2 : 1;
+    else if (long_k && kb <= 96 && t64 > 128 && t64 <= 256 &&
+             (kb + 1) / 2 * (0.45 + 0.12 * static_cast<double>(t64) / 256) < (ls.kg == 1 ? 0.9 : 1.0) * ls.cost)
+      kg = 2;
+    if (kg) {
+      p.pipe = true;
+      p.kg = kg;
+      p.bm = 64;
+      p.tiles_m = (m + 63) / 64;
+      p.tiles_n = tiles_n;
+      p.tiles = static_cast<int>(t64);
+      p.splits = 1;
+      return p;
+    }
+  }
   if (long128) p.bm = 128;
   // a single matrix with a short K and few 64-token tiles: 32-token tiles
   // give the CUs work without splitting K

@@ -73,6 +73,7 @@ struct GemmPlan {
   int tiles_m, tiles_n, tiles;
   int splits;     // workgroups per output tile along K
   bool once;      // the one-shot tile (16 or 32 tokens, K <= 2048)
+  bool pipe;      // the pipelined 32x32x16 tile (K % 64 == 0, no K split)
 };
 
 SkinnyPlan plan_skinny(int m, int k, int nmat, int tiles, bool can_split);

@@ -510,7 +510,7 @@ def test_one_shot_32_token_plan(gpu):
 
 
 @pytest.mark.parametrize("m,n,k,splits,f32", [(1800, 2000, 4160, 2, False), (1793, 2048, 4224, 2, True),
-                                              (640, 2048, 4160, 6, False), (700, 896, 4864, 8, False),
+                                              (640, 2048, 6400, 6, False), (700, 896, 4864, 8, False),
                                               (257, 2048, 4160, 8, True)])
 def test_two_k_splits_per_workgroup(gpu, m, n, k, splits, f32):
     """Long K in 128 x 128 tiles with two of the K splits in a workgroup
@@ -530,3 +530,41 @@ def test_two_k_splits_per_workgroup(gpu, m, n, k, splits, f32):
     if not f32:
         res = bf16_gpu(activations(7901, m, n), gpu)
         assert torch.equal(qw.linear(xt, bt, residual=res), res + y)
+
+
+@pytest.mark.parametrize("m,n,k,kg,f32", [(897, 2048, 2048, 2, False), (640, 2500, 2048, 2, True),
+                                          (1500, 1152, 896, 1, False), (1025, 2048, 2048, 1, False),
+                                          (1030, 2052, 64, 1, False), (1100, 1500, 128, 1, True),
+                                          (1501, 896, 4864, 2, False), (1281, 900, 4160, 2, False)])
+def test_pipelined_tiles(gpu, m, n, k, kg, f32):
+    """One round of 64 x 128 pipelined tiles (launch_pipe) with one and two K
+    groups, short and long K, one and two K steps, an odd step count over two
+    groups, ragged M and N, with bias and residual, bf16 and fp32 outputs."""
+    qw, q, s, x, b = _problem(gpu, 8100 + m + k, m, n, k, bias=True)
+    xt, bt = bf16_gpu(x, gpu), bf16_gpu(b, gpu)
+    odt = torch.float32 if f32 else torch.bfloat16
+    y = qw.linear(xt, bt, out_dtype=odt)
+    plan = _plan_kernel()
+    assert "launch_pipe" in plan and f"KG = {kg}" in plan, plan
+    rows = np.concatenate([np.random.default_rng(m).choice(m, 24, replace=False), [0, 63, 64, m - 1]])
+    report(to_np(y)[rows], O.linear(x[rows], q, s, b), k, f"pipelined m={m} n={n} k={k}",
+           acc=O.acc_bound(x[rows], q, s, b))
+    for _ in range(3):
+        assert torch.equal(y, qw.linear(xt, bt, out_dtype=odt))
+    if not f32:
+        res = bf16_gpu(activations(8101, m, n), gpu)
+        assert torch.equal(qw.linear(xt, bt, residual=res), res + y)
+
+
+def test_pipelined_group(gpu):
+    """q|k|v at 700 tokens: members of different widths in one pipelined launch."""
+    m, k = 700, 2048
+    x = activations(8200, m, k)
+    ws = [weights(8201 + j, n, k) for j, n in enumerate((2048, 256, 200))]
+    outs = Q.linear_group(bf16_gpu(x, gpu), [Q.QuantizedWeight(torch.from_numpy(w).to(gpu)) for w in ws])
+    assert "launch_pipe" in _plan_kernel(), _plan_kernel()
+    rows = np.concatenate([np.random.default_rng(1).choice(m, 24, replace=False), [0, 63, 64, m - 1]])
+    for j, w in enumerate(ws):
+        q, s = O.quantize_per_channel(w)
+        report(to_np(outs[j])[rows], O.linear(x[rows], q, s), k, f"pipelined q|k|v[{j}]",
+               acc=O.acc_bound(x[rows], q, s))

@@ -113,3 +113,24 @@ def test_pair_tiles_with_two_token_blocks(gpu, m, inter, hidden, tiled):
     ref = O.swiglu(x, *ws["gate"][1:], *ws["up"][1:])
     report(to_np(act), ref, hidden, f"pair tiles m={m} inter={inter} K={hidden}",
            acc=O.swiglu_acc(x, *ws["gate"][1:], *ws["up"][1:]))
+
+
+@pytest.mark.parametrize("m,inter,hidden,bm", [(65, 11008, 2048, 96), (96, 9000, 1024, 96), (97, 11008, 2048, 128),
+                                               (128, 16384, 64, 128), (66, 4864, 896, 64), (127, 8192, 128, 64),
+                                               (100, 130, 192, 64)])
+def test_pipelined_pair(gpu, m, inter, hidden, bm):
+    """65..128 tokens in the three pipelined tile heights: full and ragged
+    token tiles, a last tile with missing rows, one to 32 K steps."""
+    from pageserve_amd import _native
+
+    ws = _mlp_weights(gpu, 8300 + m + inter, inter, hidden)
+    x = activations(8350 + m, m, hidden)
+    xt = bf16_gpu(x, gpu)
+    act = Q.swiglu(xt, ws["gate"][0], ws["up"][0])
+    plan = _native.last_plan()
+    assert "launch_pipe" in plan and f"BM = {bm}, BN = 64" in plan, plan
+    ref = O.swiglu(x, *ws["gate"][1:], *ws["up"][1:])
+    report(to_np(act), ref, hidden, f"pipelined pair m={m} inter={inter} K={hidden}",
+           acc=O.swiglu_acc(x, *ws["gate"][1:], *ws["up"][1:]))
+    for _ in range(3):
+        assert torch.equal(act, Q.swiglu(xt, ws["gate"][0], ws["up"][0]))
