@@ -313,7 +313,7 @@ int pgs_w8a16_rmsnorm_qkv_rope(const void* x, const void* norm_weight, float eps
  * Workspace bytes a linear call needs (0 = none): n[0..n_outs-1] are the
  * out_features of its members (one member for pgs_w8a16_linear; for
  * pgs_w8a16_swiglu pass swiglu = 1 and n[0] = intermediate size).  The value
- * is exact for the same (m, n, k) and never larger than the plan needs.
+ * is fixed by the sizes and never smaller than the plan needs.
  * No counterpart in the reference, whose dense F.linear needs no workspace.
  */
 size_t pgs_w8a16_workspace_bytes(int64_t m, const int64_t* n, int n_outs,

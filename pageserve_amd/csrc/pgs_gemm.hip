@@ -1666,6 +1666,16 @@ GemmPlan plan_gemm(int m, int k, int nmat, const int32_t* n, int members, bool c
   // (without a workspace only where no partial tiles are needed, so that a
   // call plans alike with or without one)
   const bool long128 = long_k && (can_split || ls.splits == ls.kg);
+  // Workspace of a long K: room for the K split doubled until 512 workgroups,
+  // at most 8, which no plan below exceeds.  Fixed by the sizes alone, so that a
+  // workspace sized once keeps serving and the fixed-scratch entry point takes
+  // and refuses the same shapes whatever the plan.
+  if (long_k && can_split) {
+    int64_t sp = 1;
+    const int64_t tiles = tiles_for(128);
+    while (sp < 8 && tiles * sp < 512) sp *= 2;
+    if (sp > 1) p.ws_tiles = static_cast<int>(tiles * sp);
+  }
   // pipelined 64 x 128 tiles without a K split, one round of them: two K groups
   // (one workgroup per CU) for at most 256 tiles of a longer K, one group (two
   // per CU) for up to 512.  Short K: q|k|v [2560, 2048] at 640 / 768 / 1024 /
@@ -1721,8 +1731,8 @@ GemmPlan plan_gemm(int m, int k, int nmat, const int32_t* n, int members, bool c
 }
 
 size_t gemm_partial_bytes(const GemmPlan& p, int nmat) {
-  if (p.splits <= 1) return 0;
-  return static_cast<size_t>(p.tiles) * p.splits * nmat * p.bm * p.bn * sizeof(float);
+  const size_t used = p.splits <= 1 ? 0 : static_cast<size_t>(p.tiles) * p.splits * nmat * p.bm * p.bn * sizeof(float);
+  return std::max(used, static_cast<size_t>(p.ws_tiles) * 128 * 128 * sizeof(float));
 }
 
 int launch_gemm(Problem& p, const GemmPlan& plan, hipStream_t st) {

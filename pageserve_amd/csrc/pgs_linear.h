@@ -72,6 +72,7 @@ struct GemmPlan {
   int kg;         // K groups of four waves per workgroup (K % 64 == 0 kernels)
   int tiles_m, tiles_n, tiles;
   int splits;     // workgroups per output tile along K
+  int ws_tiles;  // a long K: 128 x 128 partial tiles the workspace has room for (0: as splits says)
   bool once;      // the one-shot tile (16 or 32 tokens, K <= 2048)
   bool pipe;      // the pipelined 32x32x16 tile (K % 64 == 0, no K split)
 };
