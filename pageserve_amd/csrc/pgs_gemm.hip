@@ -430,18 +430,29 @@ __device__ __forceinline__ void static_for(F&& f, std::integer_sequence<int, Js.
 
 // The same steps as whole unrolled blocks in a loop with a single exit, then
 // the remainder (fewer than sizeof...(Is) steps, positions 0, 1, ...) after
-// it.  For loops that read LDS filled by buffer-to-LDS DMA: at the head of a
-// loop with an exit after every step the compiler's wait insertion loses
-// track of which LDS object each DMA in flight targets and waits for all of
-// them; with one exit it keeps them apart.
+// it, where step takes a third argument std::true_type.  For loops that read
+// LDS filled by buffer-to-LDS DMA: at the head of a loop with an exit after
+// every step the compiler's wait insertion loses track of which LDS object
+// each DMA in flight targets and waits for all of them; with one exit it keeps
+// them apart.
 template <typename Step, int... Is>
 __device__ __forceinline__ void run_blocks(Step& step, int iters, std::integer_sequence<int, Is...>) {
   constexpr int U = sizeof...(Is);
   int j = 0;
-  for (; j + U <= iters; j += U) (step(std::integral_constant<int, Is>{}, j + Is), ...);
+  for (; j + U <= iters; j += U) (step(std::integral_constant<int, Is>{}, j + Is, std::false_type{}), ...);
   const int r = iters - j;
-  ((Is < r ? step(std::integral_constant<int, Is>{}, j + Is) : void()), ...);
+  static_for([&](auto I) { if (I < r) step(I, j + I, std::true_type{}); }, std::make_integer_sequence<int, U - 1>{});
 }
+
+// Whether position p of the remainder of a loop unrolled U times, at most
+// U - 1 steps, loads for the step `lead` ahead.  A load for a step that no
+// remainder has would be issued or not as the compiler likes (a weight load
+// without a use is deleted), so it is left out, and a counted wait knows what
+// stands behind the DMAs it waits for.
+constexpr bool tail_loads(int p, int lead, int u) { return p + lead <= u - 2; }
+
+// s_waitcnt operand for vmcnt(n) alone
+constexpr int vmcnt_only(int n) { return 0xF70 | (n & 15) | ((n >> 4) << 14); }
 
 constexpr int gcd2(int a, int b) { return b ? gcd2(b, a % b) : a; }
 constexpr int lcm3(int a, int b, int c) { return a / gcd2(a, b) * b / gcd2(a / gcd2(a, b) * b, c) * c; }
@@ -671,11 +682,11 @@ __global__ __launch_bounds__(kThreads * KG, OCC) void gemm_k64_kernel(const uint
 // own LDS object, so the compiler's LDS-DMA tracking waits for exactly the
 // DMAs of the stage a read touches; the waits that make a stage visible to
 // the other waves are explicit: every wave waits for its own DMAs of the
-// next stage (a vmcnt count: the loop issues the same loads every step),
-// then one barrier per step.  Weights go to registers as in gemm_k64_kernel.
-// Each lane's DMA writes 16 bytes at a fixed position of its wave's 1 KiB
-// slice; the lane fetches the activation piece whose swizzled home (swz) is
-// that position.
+// next stage (a vmcnt count: the loop issues the same loads every step, the
+// remainder behind it those that tail_loads says), then one barrier per step.
+// Weights go to registers as in gemm_k64_kernel.  Each lane's DMA writes 16
+// bytes at a fixed position of its wave's 1 KiB slice; the lane fetches the
+// activation piece whose swizzled home (swz) is that position.
 // 16 bytes per lane from a buffer into LDS: lane l's bytes land at lds + 16 l
 // (the LDS address is wave-uniform; it goes to M0).  A __device__ function of
 // its own: used directly in a kernel template, the builtin makes the host
@@ -817,14 +828,21 @@ __global__ __launch_bounds__(kThreads * KG, OCC) void gemm_dma_kernel(const uint
     }
   };
   // Every wave waits for its own DMAs into the stage the next step reads
-  // (issued S - 2 steps before this one; each later step issued WL weight
-  // loads, then XL DMAs), then one barrier makes the stage visible to all
-  // and frees the stage just read for the DMA of the next step.
-  constexpr int kAfter = (S - 2) * (WL + XL);
-  constexpr int kWait = 0xF70 | (kAfter & 15) | ((kAfter >> 4) << 14);
-  static_assert(kAfter < 64, "vmcnt range");
-  auto step_barrier = [&] {
-    __builtin_amdgcn_s_waitcnt(kWait);
+  // (issued S - 2 steps before this one; each later step of the loop issued WL
+  // weight loads, then XL DMAs, each later one of the remainder what
+  // tail_loads says), then one barrier makes the stage visible to all and
+  // frees the stage just read for the DMA of the next step.  A count that
+  // includes a load which is not issued leaves DMAs of that stage in flight
+  // at the barrier.
+  static_assert((S - 2) * (WL + XL) < 64, "vmcnt range");
+  constexpr auto younger = [](int i, bool tail) {
+    int n = 0;
+    for (int t = i - (S - 3); t <= i; ++t)
+      n += !tail || t < 0 ? WL + XL : (tail_loads(t, WLEAD, UNROLL) ? WL : 0) + (tail_loads(t, S - 1, UNROLL) ? XL : 0);
+    return n;
+  };
+  auto step_barrier = [&](auto AFTER) {
+    __builtin_amdgcn_s_waitcnt(vmcnt_only(decltype(AFTER)::value));
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
@@ -834,29 +852,32 @@ __global__ __launch_bounds__(kThreads * KG, OCC) void gemm_dma_kernel(const uint
   // set (i + WLEAD) % WSETS, DMA of j + S - 1 into stage (i + S - 1) % S
   // (loads past the last step repeat it: in bounds, counts unchanged), the
   // MFMAs of j on set i % WSETS and stage i % S, then the barrier.
-  auto step = [&](auto I, int j) {
+  auto step = [&](auto I, int j, auto TAIL) {
     constexpr int i = decltype(I)::value;
+    constexpr bool tail = decltype(TAIL)::value;
     const int kt = first + j * KG;
-    wload(min(kt + WLEAD * KG, last), wset[(i + WLEAD) % WSETS]);
-    dma(stage(std::integral_constant<int, (i + S - 1) % S>{}), min(kt + (S - 1) * KG, last));
+    if constexpr (!tail || tail_loads(i, WLEAD, UNROLL)) wload(min(kt + WLEAD * KG, last), wset[(i + WLEAD) % WSETS]);
+    if constexpr (!tail || tail_loads(i, S - 1, UNROLL))
+      dma(stage(std::integral_constant<int, (i + S - 1) % S>{}), min(kt + (S - 1) * KG, last));
     __builtin_amdgcn_sched_barrier(0);
     __builtin_amdgcn_s_setprio(1);
     if (KG == 1 || kt < kt1) compute(wset[i % WSETS], stage(std::integral_constant<int, i % S>{}));
     __builtin_amdgcn_s_setprio(0);
-    step_barrier();
+    step_barrier(std::integral_constant<int, younger(i, tail)>{});
   };
   // (the planner gives every split at least one K step; a guard on iters here
   // costs the accumulators their registers: the compiler then spills them)
   {
     // prologue: stages 0 .. S-2, then weights 0 .. WLEAD-1; wait for stage 0
+    // (in this order: the count below relies on it)
     static_for([&](auto J) { dma(stage(J), min(first + decltype(J)::value * KG, last)); },
                std::make_integer_sequence<int, S - 1>{});
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int j = 0; j < WLEAD; ++j) wload(min(first + j * KG, last), wset[j]);
     constexpr int kPro = (S - 2) * XL + WLEAD * WL;
-    constexpr int kProWait = 0xF70 | (kPro & 15) | ((kPro >> 4) << 14);
     static_assert(kPro < 64, "vmcnt range");
-    __builtin_amdgcn_s_waitcnt(kProWait);
+    __builtin_amdgcn_s_waitcnt(vmcnt_only(kPro));
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
     run_blocks(step, iters, std::make_integer_sequence<int, UNROLL>{});
@@ -1061,7 +1082,7 @@ __global__ __launch_bounds__(64 * NW * KG, OCC) void gemm_pipe_kernel(const uint
   constexpr int kAfter = (S - 4) * OPS + n012;
   constexpr int kWait = 0xF70 | (kAfter & 15) | ((kAfter >> 4) << 14);
   static_assert(kAfter < 64, "vmcnt range");
-  auto step = [&](auto I, int j) {
+  auto step = [&](auto I, int j, auto) {
     constexpr int i = decltype(I)::value;
     const int kt = kg + j * KG;
     const int ktw = min(kt + WLEAD * KG, last), ktx = min(kt + (S - 1) * KG, last);
