@@ -938,9 +938,8 @@ __global__ __launch_bounds__(kThreads * KG, OCC) void gemm_dma_kernel(const uint
 //    the B fragments of c + 1 are read, its weights are widened and a share of
 //    the step's loads is issued between the MFMAs, the first sub-step of the
 //    next step included: the step's barrier stands before the last sub-step.
-//  * S stages of activations by LDS DMA; a stage is waited for one whole step
-//    before its first read (a read right behind the wait and the barrier has
-//    returned stale data here with stages written by other waves' DMAs).
+//  * S stages of activations by LDS DMA; a stage is waited for at the barrier
+//    one whole step before its first read.
 //  * KG = 2: two groups of NW waves on alternate K steps, as in gemm_dma_kernel.
 //  * The epilogue's scales, bias and residuals are loaded before the loop.
 // Wave (wn, wm) of a group owns BN / (NW / WM) rows of each matrix and BM / WM
@@ -1074,16 +1073,24 @@ __global__ __launch_bounds__(64 * NW * KG, OCC) void gemm_pipe_kernel(const uint
     }
   };
   // A step issues its weight loads, then its DMAs, spread over the MFMAs: load
-  // o behind MFMA o * SLOTS / OPS.  At its barrier, behind the third sub-step,
-  // each wave has waited for its own DMAs of the stage two steps on (issued
-  // S - 3 steps ago; n012 of this step's loads are younger, and all of each
-  // step between).
+  // o behind MFMA o * SLOTS / OPS (in the remainder those that tail_loads
+  // says).  At its barrier, behind the third sub-step, each wave has waited for
+  // its own DMAs of the stage two steps on (issued S - 3 steps ago; the first
+  // n012 of this step's loads are younger, and all of each step between).
   constexpr int n012 = (3 * TB * OPS + SLOTS - 1) / SLOTS;
-  constexpr int kAfter = (S - 4) * OPS + n012;
-  constexpr int kWait = 0xF70 | (kAfter & 15) | ((kAfter >> 4) << 14);
-  static_assert(kAfter < 64, "vmcnt range");
-  auto step = [&](auto I, int j, auto) {
+  static_assert(WLEAD >= S - 4 && (S - 4) * OPS + n012 < 64, "vmcnt range");
+  constexpr auto issued = [](int p, bool tail, int o) {  // load o of the step at position p
+    return !tail || p < 0 || tail_loads(p, o < WL ? WLEAD : S - 1, UNROLL);
+  };
+  constexpr auto younger = [issued](int i, bool tail) {
+    int n = 0;
+    for (int t = i - (S - 4); t <= i; ++t)
+      for (int o = 0; o < (t < i ? OPS : n012); ++o) n += issued(t, tail, o);
+    return n;
+  };
+  auto step = [&](auto I, int j, auto TAIL) {
     constexpr int i = decltype(I)::value;
+    constexpr bool tail = decltype(TAIL)::value;
     const int kt = kg + j * KG;
     const int ktw = min(kt + WLEAD * KG, last), ktx = min(kt + (S - 1) * KG, last);
     const bool on = KG == 1 || kt < kb;
@@ -1108,14 +1115,14 @@ __global__ __launch_bounds__(64 * NW * KG, OCC) void gemm_pipe_kernel(const uint
         }
 #pragma unroll
         for (int o = 0; o < OPS; ++o)
-          if (o * SLOTS / OPS == c * TB + jj) {
+          if (o * SLOTS / OPS == c * TB + jj && issued(i, tail, o)) {
             if (o < WL) wload1(o, ktw, wl);
             else dma1(fill, o - WL, ktx);
           }
         __builtin_amdgcn_sched_barrier(0);
       }
       if (c == 2) {
-        __builtin_amdgcn_s_waitcnt(kWait);
+        __builtin_amdgcn_s_waitcnt(vmcnt_only(younger(i, tail)));
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
@@ -1137,9 +1144,8 @@ __global__ __launch_bounds__(64 * NW * KG, OCC) void gemm_pipe_kernel(const uint
       for (int o = 0; o < WL; ++o) wload1(o, min(kg + j * KG, last), wset[j]);
     __builtin_amdgcn_sched_barrier(0);
     constexpr int kPro = (S - 3) * XL + WLEAD * WL;
-    constexpr int kProWait = 0xF70 | (kPro & 15) | ((kPro >> 4) << 14);
     static_assert(kPro < 64, "vmcnt range");
-    __builtin_amdgcn_s_waitcnt(kProWait);
+    __builtin_amdgcn_s_waitcnt(vmcnt_only(kPro));
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
     pair_operand(wset[0]);

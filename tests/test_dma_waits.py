@@ -7,7 +7,8 @@ value is never used is deleted.  So the built code is replayed here, on the
 CPU: along every path through a kernel, the vector memory operations in issue
 order, the waits (they complete in order) and the barriers.  A wave's DMAs fill
 one K step's stage after the other, `per_stage` of them each, and barrier k
-stands in front of the reads of step k's stage.
+stands in front of the reads of step k's stage.  gemm_pipe_kernel promises more:
+barrier k hands over the stage of step k + 1 (`lead` = 1).
 """
 
 from __future__ import annotations
@@ -70,15 +71,15 @@ def events(code):
     return ev, labels
 
 
-def uncovered(code, per_stage: int, closing: int) -> set[tuple[int, int]]:
+def uncovered(code, per_stage: int, closing: int, lead: int = 0) -> set[tuple[int, int]]:
     """(event, missing DMAs) of barriers that hand over a stage some of whose
     DMAs may be in flight.  The state of a path: the operations in flight in
     issue order, the DMAs landed beyond those of the stages handed over, and
     the barriers that left some missing, each with how many more barriers show
-    that a step followed it (the path ends with `closing` barriers that hand
-    over no stage)."""
+    that the step it should have served followed (the path ends with `closing`
+    barriers that hand over no stage)."""
     ev, labels = events(code)
-    bad, seen, todo = set(), set(), [(0, (), 0, ())]
+    bad, seen, todo = set(), set(), [(0, (), -lead * per_stage, ())]
     while todo:
         state = todo.pop()
         if state in seen:
@@ -97,7 +98,7 @@ def uncovered(code, per_stage: int, closing: int) -> set[tuple[int, int]]:
             ahead -= per_stage
             short = tuple((a, n, left - 1) for a, n, left in short if left > 1)
             if ahead < 0:
-                short += ((at, -ahead, closing + 1),)
+                short += ((at, -ahead, closing + lead + 1),)
         if kind == "s_endpgm":
             continue
         if arg in labels:
@@ -115,9 +116,8 @@ def tile_kernels(native_lib, tmp_path_factory):
 
 
 def test_stages_are_waited_for(tile_kernels):
-    """gemm_dma_kernel: every remainder length of its unrolled K loop, the loop
-    entered or not."""
-    faults, count = {}, {"dma": 0}
+    """Every remainder length of the unrolled K loop, the loop entered or not."""
+    faults, count = {}, {"dma": 0, "pipe": 0}
     for name, code in tile_kernels.items():
         kind, args = re.match(r"gemm_(\w+)_kernel<(.*)>", name).groups()
         if kind not in count:
@@ -127,10 +127,10 @@ def test_stages_are_waited_for(tile_kernels):
         bm, kg = p[0], p[-1] if kind == "dma" else p[3]
         waves = 4 if kind == "dma" else p[4]
         # (two K groups exchange their sums in two halves, two barriers each)
-        bad = uncovered(code, bm * 8 // (64 * waves), 4 if kg == 2 else 0)
+        bad = uncovered(code, bm * 8 // (64 * waves), 4 if kg == 2 else 0, lead=kind == "pipe")
         if bad:
             faults[name] = sorted(bad)
-    assert count == {"dma": 8}, count
+    assert count == {"dma": 8, "pipe": 7}, count
     assert not faults, faults
 
 

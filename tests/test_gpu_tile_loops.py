@@ -44,7 +44,7 @@ def _check(gpu, plan, pair, m, n, k, f32):
     assert ok, (k // 64, int((y.double() - ref).abs().gt(2.0**-8 * ref.abs() + 1e-6).sum()))
 
 
-DMA = [
+CASES = [
     # unrolled by 3: the pair in 128-token tiles, lm_head's 128 x 128, 64 x 128
     ("gemm_dma", "BM = 128, BN = 64, NMAT = 2", True, 250, 200, range(1, 9)),
     ("gemm_dma", "BM = 128, BN = 128, NMAT = 1", False, 256, 131072, range(1, 7)),
@@ -53,10 +53,18 @@ DMA = [
     ("gemm_dma", "BM = 64, BN = 64, NMAT = 2", True, 160, 200, range(1, 11)),
     # two K groups: even and odd numbers of steps, 33 .. 36 in a group
     ("gemm_dma", "KG = 2", False, 1800, 2000, range(65, 72)),
+    # the pipelined pair, unrolled by 5
+    ("gemm_pipe", "BM = 64, BN = 64, NMAT = 2", True, 100, 200, range(1, 12)),
+    ("gemm_pipe", "BM = 96, BN = 64, NMAT = 2", True, 90, 8200, range(1, 12)),
+    ("gemm_pipe", "BM = 128, BN = 64, NMAT = 2", True, 128, 8200, range(1, 12)),
+    # the pipelined 64 x 128 tile, unrolled by 12 (each count in both output
+    # types), and its two K groups (17 .. 28 steps in a group)
+    ("gemm_pipe", "KG = 1", False, 1024, 1600, [kb for kb in range(1, 26) for _ in "ab"]),
+    ("gemm_pipe", "KG = 2", False, 1024, 1600, range(33, 57)),
 ]
 
 
-@pytest.mark.parametrize("kernel,plan,pair,m,n,steps", DMA, ids=[c[1] for c in DMA])
+@pytest.mark.parametrize("kernel,plan,pair,m,n,steps", CASES, ids=[f"{c[0]} {c[1]}" for c in CASES])
 def test_every_remainder_of_the_k_loop(gpu, kernel, plan, pair, m, n, steps):
     for i, kb in enumerate(steps):
         print(plan, "K steps", kb, flush=True)
