@@ -236,10 +236,11 @@ def _chain(attn, residual, o, ln_post, gate, up, down, eps, next_ln, next_qkv, n
     x = Q.rmsnorm_mlp(x1, ln_post, eps, gate, up, down, residual=x1)
     if next_qkv is None:
         return x, None
+    biases = list(next_bias) if next_bias else None  # (an empty list: no biases)
     if (cos is not None and x.numel() and head_dim % 2 == 0 and 2 <= head_dim <= 65536
             and all(w.shape[0] > 0 and w.shape[0] % head_dim == 0 for w in next_qkv[:2]) and next_qkv[2].shape[0] > 0):
-        return x, tuple(Q._rmsnorm_qkv_rope(x, next_ln, eps, list(next_qkv), next_bias, cos, sin, head_dim))
-    q, k, v = Q.rmsnorm_linear_group(x, next_ln, eps, list(next_qkv), list(next_bias) if next_bias else None)
+        return x, tuple(Q._rmsnorm_qkv_rope(x, next_ln, eps, list(next_qkv), biases, cos, sin, head_dim))
+    q, k, v = Q.rmsnorm_linear_group(x, next_ln, eps, list(next_qkv), biases)
     if cos is not None:
         m = q.shape[0] if q.dim() == 2 else q.numel() // q.shape[-1]
         q3 = q.reshape(m, -1, head_dim)

@@ -10,6 +10,7 @@ import torch
 
 import pageserve_amd
 from pageserve_amd import quantization as Q
+from pageserve_amd import span
 
 
 def test_reference_api_surface():
@@ -64,3 +65,43 @@ def test_linear_requires_a_gpu_resident_weight():
         Q.linear(torch.zeros(1, 16, dtype=torch.bfloat16), Fake())
     with pytest.raises(ValueError, match="1..4"):
         Q.linear_group(torch.zeros(1, 16, dtype=torch.bfloat16), [])
+
+
+class _Weight:
+    """A weight as the fused calls see it, its packed bytes on the CPU."""
+
+    def __init__(self, n, k, cuda):
+        self.shape = torch.Size((n, k))
+        self.qp = type("Packed", (), {"is_cuda": cuda})()
+        self._operands = (torch.zeros(1, dtype=torch.int8), torch.zeros(n), n, k, torch.device("cpu"))
+
+    def _launch_operands(self):
+        return self._operands
+
+
+def _chain_tail(monkeypatch, cuda, next_bias):
+    """decode_span's per-projection chain with RoPE, its MLP and its q|k|v
+    launch taken out; the biases that the launch was given."""
+    m, k, hd = 2, 64, 32
+    x = torch.zeros(m, k, dtype=torch.bfloat16)
+    seen = []
+
+    class Host:
+        @staticmethod
+        def qkv_rope(x, qs, ss, biases, ns, *rest):
+            seen.append(biases)
+            return [torch.zeros(m, n, dtype=torch.bfloat16) for n in ns]
+
+    monkeypatch.setattr(Q._native, "load_host", lambda: Host)
+    monkeypatch.setattr(Q, "_ws_args", lambda *a: (0, 0, None))
+    monkeypatch.setattr(Q, "rmsnorm_mlp", lambda x, *a, **kw: x)
+    o = type("O", (), {"linear": staticmethod(lambda a, residual: a)})
+    cs = torch.zeros(m, hd, dtype=torch.bfloat16)
+    qkv = [_Weight(n, k, cuda) for n in (64, 32, 32)]
+    span._chain(x, x, o, None, None, None, None, 1e-6, torch.ones(k), qkv, next_bias, cs, cs, hd)
+    return seen[0]
+
+
+@pytest.mark.parametrize("none", [None, (), []])
+def test_decode_chain_takes_empty_biases_as_none(monkeypatch, none):
+    assert _chain_tail(monkeypatch, True, none) == [None, None, None]
