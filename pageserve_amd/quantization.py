@@ -592,6 +592,8 @@ def _rmsnorm_qkv_rope(x, norm_weight, eps, weights, biases, cos, sin, head_dim) 
     first two (engine/model.py:166-173), in one launch where the norm runs
     inside the projection and the heads allow it.  ``q`` and ``k`` must be
     whole heads of ``head_dim``."""
+    if not weights[0].qp.is_cuda:
+        raise RuntimeError("W8A16 linear: the weight must be on a ROCm GPU (call .to('cuda') first)")
     ops = [w._launch_operands() for w in weights]
     _, _, _, k, dev = ops[0]
     if any(o[3] != k or o[4] != dev for o in ops):

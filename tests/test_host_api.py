@@ -105,3 +105,8 @@ def _chain_tail(monkeypatch, cuda, next_bias):
 @pytest.mark.parametrize("none", [None, (), []])
 def test_decode_chain_takes_empty_biases_as_none(monkeypatch, none):
     assert _chain_tail(monkeypatch, True, none) == [None, None, None]
+
+
+def test_decode_chain_says_where_its_weights_belong(monkeypatch):
+    with pytest.raises(RuntimeError, match=r"ROCm GPU \(call .to\('cuda'\) first\)"):
+        _chain_tail(monkeypatch, False, None)
