@@ -81,10 +81,10 @@ SkinnyPlan plan_skinny(int m, int k, int nmat, int tiles, bool can_split);
 // workgroups of a skinny launch
 int64_t skinny_grid(const SkinnyPlan& p);
 size_t skinny_partial_bytes(const SkinnyPlan& p, int nmat);
-// whether the skinny kernel can apply rms_norm to its staged activations
-// (bf16 output, K % 64 == 0, no K split, an issue-once shape whose registers
-// and LDS hold it)
-bool skinny_norm_fusable(const SkinnyPlan& p, int m, int k, bool out_f32, int nmat);
+// whether the skinny kernel applies rms_norm to the activations it loads (bf16
+// output, K % 64 == 0, no K split, an issue-once shape whose registers and LDS
+// hold it, few enough row tiles); rope: the launch then rotates too
+bool skinny_norm_fusable(const SkinnyPlan& p, int m, int k, bool out_f32, int nmat, bool rope);
 // whether a launch with the fused norm can also rotate its first two members
 // (unfolded tiles; whole heads of a multiple of 32 dimensions)
 bool skinny_rope_fusable(const SkinnyPlan& p, int hd, const GroupArgs& a);

@@ -82,7 +82,9 @@ int run(Problem& p, void* workspace, size_t ws_bytes, hipStream_t st) {
   const int members = (p.nmat == 2) ? 1 : p.args.n_outs;
   const Plan plan = make_plan(p.m, p.k, p.nmat, p.args.n, members, workspace != nullptr);
   const size_t need = workspace_bytes(plan, p.nmat);
-  if (p.norm_w && !(plan.skinny && skinny_norm_fusable(plan.sk, p.m, p.k, p.out_f32, p.nmat) && aligned(p.norm_w, 16))) {
+  const bool rope = p.rope_cos && plan.skinny && skinny_rope_fusable(plan.sk, p.rope_hd, p.args);
+  if (p.norm_w && !(plan.skinny && skinny_norm_fusable(plan.sk, p.m, p.k, p.out_f32, p.nmat, rope) &&
+                    aligned(p.norm_w, 16))) {
     // rms_norm as its own kernel into the workspace, then the plain linear
     const size_t off = norm_offset(need), bytes = static_cast<size_t>(p.m) * p.k * 2;
     if (!workspace || ws_bytes < off + bytes)
@@ -95,7 +97,7 @@ int run(Problem& p, void* workspace, size_t ws_bytes, hipStream_t st) {
     p.norm_w = nullptr;
     ws_bytes = off;
   }
-  if (p.rope_cos && !(p.norm_w && skinny_rope_fusable(plan.sk, p.rope_hd, p.args))) {
+  if (p.rope_cos && !(p.norm_w && rope)) {
     // RoPE as its own kernel, in place on the projections' outputs
     Problem lin = p;
     lin.rope_cos = lin.rope_sin = nullptr;

@@ -109,16 +109,19 @@ constexpr int skinny_lds_bytes(int nw, int u, int nb, int nmat, int s, int xm, b
 constexpr int norm_xm(int m) { return m <= 1 ? 1 : m <= 2 ? 2 : m <= 4 ? 4 : m <= 8 ? 8 : m <= 16 ? 16 : 0; }
 // Whether a launch shape has the fused norm for that many staged tokens: above
 // four tokens a lane keeps its activations and norm weights in registers beside
-// its weight loads, which fits for at most four slots per wave (K <= 2048 with
-// eight waves, 4096 with sixteen).  The SwiGLU pair has it up to four tokens: its
-// several workgroups per CU would each repeat the norm (6 / 12 / 24 tokens cost
-// 2.9 / 5.5 / 14 us more, against 3.3 / 3.5 / 4.3 for the norm as a launch).
+// its weight loads, which fits for at most four slots per wave of at most eight
+// waves (K <= 2048; sixteen waves, K up to 4096, cost more than the norm's own
+// launch: [4096 | 1024 | 1024, 4096] at 5 / 16 tokens 13.9 / 20.1 us against
+// 10.0 / 13.6).  The SwiGLU pair has it up to four tokens: its several
+// workgroups per CU would each repeat the norm (6 / 12 / 24 tokens cost 2.9 /
+// 5.5 / 14 us more, against 3.3 / 3.5 / 4.3 for the norm as a launch).
 constexpr bool norm_shape(int nw, int u, int nb, int nmat, bool fold, int xm) {
   const int s = fold ? 2 : 1;
   if (nb == 0 || (nmat == 2 && (xm == 0 || xm > 4))) return false;
   if (xm == 0) return !fold && nw == 8 && nb == 2;
   if (xm == 16 && fold) return false;
-  return (xm <= 4 || u * nb * s <= 4) && skinny_lds_bytes(nw, u, nb, nmat, s, xm, true) + nw * u * nb * s * 128 <= kLdsLimit;
+  return (xm <= 4 || (nw <= 8 && u * nb * s <= 4)) &&
+         skinny_lds_bytes(nw, u, nb, nmat, s, xm, true) + nw * u * nb * s * 128 <= kLdsLimit;
 }
 
 // Eight bf16 activations after rms_norm with row factor r and eight norm
@@ -1055,8 +1058,30 @@ SkinnyPlan plan_skinny(int m, int k, int nmat, int tiles, bool can_split) {
   return p;
 }
 
-bool skinny_norm_fusable(const SkinnyPlan& p, int m, int k, bool out_f32, int nmat) {
-  if (out_f32 || m < 1 || m > 32 || k % 64 != 0 || p.splits != 1 || p.pair) return false;
+// Row tiles up to which a launch takes the norm inside.  Above four tokens every
+// workgroup repeats the norm, at a cost that grows with the workgroups per CU and
+// with K (eight waves instead of four above 1024), while the launches saved cost
+// the same at any size: the norm's, and the rotation's where the launch then rotates too.
+// Measured, time with the norm inside over time with it as a launch (the whole
+// call: norm, projections and, where named, RoPE; K = 256 .. 2048, 8 .. 2000 tiles):
+//   5..8 tokens, K <= 1024: 0.69 .. 0.94 up to 1024 tiles, 0.95 .. 1.14 at 2000;
+//     longer K: 0.93 up to 256, 0.96 .. 1.05 at 320..512, 1.2 at 1024; with RoPE
+//     0.71 .. 0.85 up to 512, 0.9 at 688, 1.06 at 1024
+//   9..16 tokens, K <= 1024: 0.78 .. 0.98 up to 512, 0.92 .. 1.06 at 688, 1.1 at
+//     1024; longer K: 1.06 .. 1.11 from 160 on; with RoPE 0.82 .. 0.89 up to 256,
+//     0.95 .. 1.02 at 320..512, 1.2 at 688
+//   17..32 tokens (two token blocks): 1.1 and more at any count; with RoPE 0.90 ..
+//     1.0 up to 256, 1.25 .. 1.39 at 320
+static int norm_tiles(int m, int k, bool rope) {
+  if (m <= 4) return 0x7fffffff;
+  if (m <= 8) return k <= 1024 ? 1024 : rope ? 512 : 256;
+  if (m <= 16) return k <= 1024 ? 512 : rope ? 256 : 0;
+  return rope ? 256 : 0;
+}
+
+bool skinny_norm_fusable(const SkinnyPlan& p, int m, int k, bool out_f32, int nmat, bool rope) {
+  if (out_f32 || m < 1 || m > 32 || k % 64 != 0 || p.splits != 1 || p.pair || p.tiles > norm_tiles(m, k, rope))
+    return false;
   const SkinnyShape& sh = kSkinnyShapes[p.shape];
   return norm_shape(sh.nw, sh.u, sh.nb, nmat, p.fold, norm_xm(m));
 }

@@ -250,3 +250,29 @@ def test_qkv_rope_of_random_rows_matches_oracle(gpu):
         h, dh = O.rmsnorm(x, w, eps), O.rmsnorm_dx(x, w, eps)
         for o, (q, s) in zip(outs, qs):
             report(to_np(o), O.linear(h, q, s), k, f"qkv_rope m={m}", acc=O.acc_bound(h, q, s, dx=dh))
+
+
+# both sides of every limit on the row tiles, and K = 4096 (sixteen waves)
+@pytest.mark.parametrize("m,k,tiles,rope,inside", [
+    (8, 1024, 1024, False, True), (8, 1024, 1040, False, False), (8, 2048, 256, False, True), (5, 2048, 272, False, False),
+    (8, 2048, 512, True, True), (8, 2048, 528, True, False), (16, 1024, 512, False, True), (9, 1024, 528, False, False),
+    (9, 2048, 144, False, False), (16, 2048, 256, True, True), (9, 2048, 272, True, False), (17, 896, 144, False, False),
+    (32, 2048, 256, True, True), (17, 896, 272, True, False), (8, 4096, 256, True, False), (5, 4096, 256, False, False)])
+def test_norm_inside_up_to_a_number_of_row_tiles(gpu, m, k, tiles, rope, inside):
+    """Many workgroups each repeating the norm cost more than its launch: the
+    route, and the same result as the separate calls on either."""
+    hd = 64
+    _, qws, _ = group(gpu, k + tiles, [tiles * 16 - 128, 64, 64], k)
+    x = bf16_gpu(exact_sum_inputs(m + tiles, m, k), gpu)
+    w = bf16_gpu(norm_weight(k + 4, k), gpu)
+    cos, sin = (bf16_gpu(norm_weight(m + j, m * hd).reshape(m, hd), gpu) for j in range(2))
+    ref = Q.linear_group(Q.rmsnorm(x, w, 1e-6), qws)
+    if rope:
+        out = Q._rmsnorm_qkv_rope(x, w, 1e-6, qws, None, cos, sin, hd)
+        for y in ref[:2]:
+            y3 = y.view(m, -1, hd)
+            Q.rope_qk(y3, None, cos, sin, inplace=True)
+    else:
+        out = Q.rmsnorm_linear_group(x, w, 1e-6, qws)
+    assert ("NORM = true" in _native.last_plan()) == inside, _native.last_plan()
+    assert all(torch.equal(a, b) for a, b in zip(out, ref))
