@@ -837,15 +837,17 @@ int launch_shape(Problem& p, const SkinnyPlan& plan, hipStream_t st) {
 
 // The SwiGLU pair at 14..32 tokens with a short K (K % 64 == 0, at most
 // NW * CPW chunks): RT row tiles per workgroup instead of one.  With one tile
-// per workgroup every workgroup loads the tokens'
-// whole activation rows for its 16 rows, as many bytes as its weights at 16
-// tokens and twice as many at 32; here each activation fragment feeds the RT
-// tiles' gate and up MFMAs, and RT = ceil(tiles / 256) gives at most one
-// workgroup per CU (230 for an 11008-row pair).  Wave w takes chunks w * CPW ..
-// w * CPW + CPW - 1 of every tile and issues all of its loads at once (one
-// memory round trip), the activations first; the waves' partial tiles are
-// summed through LDS in wave order (a fixed order: reproducible), then each
-// output thread applies silu(g s_g)(u s_u) (engine/model.py:188-189).
+// per workgroup every workgroup loads the tokens' whole activation rows for its
+// 16 rows, as many bytes as its weights at 16 tokens and twice as many at 32;
+// here each activation fragment feeds the RT tiles' gate and up MFMAs, two where
+// that gives at most one workgroup per CU, else three (230 for an 11008-row
+// pair).  Wave w takes chunks w * CPW .. w * CPW + CPW - 1 of every tile and
+// issues all of its loads at once (one memory round trip): with two token blocks
+// the activations first, with one behind each chunk's weights (activations first
+// 9.60 against 9.10 us at 8960 x 1536 and 16 tokens, 4 % up to 20000 rows).  The
+// waves' partial tiles are summed through LDS in wave order (a fixed order:
+// reproducible), then each output thread applies silu(g s_g)(u s_u)
+// (engine/model.py:188-189).
 // Measured on the 11008 x 2048 pair (us, one-tile plan -> this kernel): 16
 // tokens 11.56 -> 11.20, 14: 11.15 -> 11.02, but 13: 11.0 -> 11.1 and 9: 10.1 ->
 // 10.5 (sixteen waves of two chunks); two token blocks (eight waves of four
@@ -895,22 +897,35 @@ __global__ __launch_bounds__(64 * NW, 1) void pair_tiles_kernel(const uint16_t* 
     }
   };
   u32x4 w[CPW][RT][2], xb[CPW][TM][2];
-#pragma unroll
-  for (int j = 0; j < CPW; ++j)
+  auto load_x = [&](int j) {
 #pragma unroll
     for (int t = 0; t < TM; ++t) {
       xb[j][t][0] = __builtin_amdgcn_raw_buffer_load_b128(xres, xoff[t], (wave * CPW + j) * 128, 0);
       xb[j][t][1] = __builtin_amdgcn_raw_buffer_load_b128(xres, xoff[t] + 16, (wave * CPW + j) * 128, 0);
     }
-  __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-  for (int j = 0; j < CPW; ++j)
+  };
+  auto load_w = [&](int j) {
 #pragma unroll
     for (int r = 0; r < RT; ++r)
 #pragma unroll
       for (int mat = 0; mat < 2; ++mat)
         w[j][r][mat] = __builtin_amdgcn_raw_buffer_load_b128(wres[r][mat], lane * 16, (wave * CPW + j) * 1024, kLoadNT);
-  __builtin_amdgcn_sched_barrier(0);  // every load issued before the first wait
+  };
+  if constexpr (TM == 1) {
+    load_scales();
+#pragma unroll
+    for (int j = 0; j < CPW; ++j) {
+      load_w(j);
+      load_x(j);
+    }
+  } else {
+#pragma unroll
+    for (int j = 0; j < CPW; ++j) load_x(j);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int j = 0; j < CPW; ++j) load_w(j);
+    __builtin_amdgcn_sched_barrier(0);  // every load issued before the first wait
+  }
   // a chunk past K reads zero weights; its activations (the next token's
   // row, or zeros) are masked too, so non-finite values cannot leak in
 #pragma unroll
@@ -922,7 +937,7 @@ __global__ __launch_bounds__(64 * NW, 1) void pair_tiles_kernel(const uint16_t* 
       xb[j][t][1] &= mask;
     }
   }
-  load_scales();
+  if constexpr (TM == 2) load_scales();
   f32x4 acc[RT][2][TM];
 #pragma unroll
   for (int r = 0; r < RT; ++r)
