@@ -987,7 +987,13 @@ __global__ __launch_bounds__(64 * NW, 1) void pair_tiles_kernel(const uint16_t* 
 
 // The launch of pair_tiles_kernel a SwiGLU pair takes at these sizes: row
 // tiles per workgroup (0: none), waves and chunks per wave.  Two token blocks
-// only where one round of workgroups fills more than half of the CUs.
+// only where one round of workgroups fills more than half of the CUs, and with
+// four chunks per wave only from the tokens on whose activation loads outweigh
+// the longer chain of a workgroup, the more rounds the one-tile plan has (K = 2048,
+// one-tile plan -> this kernel: 560 tiles at 17 tokens 11.81 -> 11.77 us; 625 at
+// 17 / 19 12.09 / 12.26 -> 12.26 / 12.16; 688 at 17 / 20 / 22 11.96 / 12.86 /
+// 13.28 -> 12.51 / 12.82 / 12.86; 768 at 18 / 20 / 24 12.29 / 12.96 / 14.06 ->
+// 13.22 / 13.51 / 14.14; K = 1536, 750 at 17 / 20 11.93 / 12.82 -> 11.97 / 12.29).
 struct PairTiles {
   int rt, nw, cpw;
 };
@@ -995,6 +1001,7 @@ PairTiles pair_tiles(int m, int k, const SkinnyPlan& plan) {
   if (plan.splits != 1 || k % 64 != 0 || k > 2048) return {0, 0, 0};
   if (m < 14 || m > 32) return {0, 0, 0};
   if (m > 16 && (plan.tiles <= 256 || plan.tiles > 768)) return {0, 0, 0};
+  if (m > 16 && k > 1536 && m <= 16 + (plan.tiles - 560) / 26) return {0, 0, 0};
   const int rt = plan.tiles > 256 && plan.tiles <= 512 ? 2 : 3;
   if (k <= 1024) return {rt, 8, 2};
   return m <= 16 ? PairTiles{rt, 16, 2} : PairTiles{rt, 8, 4};

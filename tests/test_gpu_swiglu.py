@@ -99,11 +99,14 @@ def test_pair_tiles_plan(gpu):
 
 @pytest.mark.parametrize("m,inter,hidden,tiled", [(17, 4112, 2048, True), (32, 8192, 1024, True), (31, 8208, 1088, True),
                                                   (24, 12288, 64, True), (20, 4096, 512, False),
-                                                  (18, 12304, 128, False), (25, 5000, 896, True)])
+                                                  (18, 12304, 128, False), (25, 5000, 896, True),
+                                                  (20, 11008, 2048, False), (21, 11008, 2048, True),
+                                                  (24, 12288, 1600, False), (25, 12288, 1600, True)])
 def test_pair_tiles_with_two_token_blocks(gpu, m, inter, hidden, tiled):
     """17..32 tokens at the edges of the two- and three-tile plans (257, 512,
     513 and 768 row tiles; 16 and 17 chunks) and just outside them, a last
-    workgroup with missing tiles and a last tile with missing rows."""
+    workgroup with missing tiles and a last tile with missing rows, and the
+    token counts at which many tiles of a longer K begin."""
     from pageserve_amd import _native
 
     ws = _mlp_weights(gpu, 700 + m + inter, inter, hidden)
