@@ -299,6 +299,23 @@ int launch_dequant(const int8_t* q, const float* scale, int64_t n, int64_t k, vo
   return check_launch("pgs_dequantize");
 }
 
+// Whether the eight-row kernel is the faster one.  Its workgroups hold eight rows
+// and wait for all of a row's loads, so it needs about one per CU; below that the
+// n workgroups of the one-row kernel, small and read from L2 the second time, end
+// sooner (one-row -> eight-row kernel, us).  Row-major fp32 [n, 2048] at n = 256 /
+// 1024 / 1536 / 4096: 3.0 -> 4.2, 4.4 -> 4.7, 5.3 -> 5.3, 10.9 -> 9.0, and [n, 8192]
+// at 256 / 1024 / 1536: 6.7 -> 10.7, 12.3 -> 12.8, 18.4 -> 15.4; bf16 [n, 2048] at
+// 1024 / 2048 / 4096: 3.8 -> 4.2, 5.0 -> 5.1, 7.6 -> 7.1.  Packed, whose one-row kernel
+// writes parts of lines: fp32 [n, 2048] at 256 / 1024: 3.4 -> 4.4, 5.4 -> 4.9, [n,
+// 12288] at 256 / 512: 10.7 -> 12.8, 16.6 -> 14.1.  Where padding is to be cleared the
+// one-row kernel needs a fill launch: [150, 2048] 4.7 -> 4.1, only longer rows are
+// sooner done with it ([300 | 600, 8192] 10.2 -> 11.0, 13.9 -> 11.8).
+bool tile_quantizer(bool packed, bool f32, int64_t n, int64_t k) {
+  if (packed && (n % 16 != 0 || k % 64 != 0)) return k <= 5120 || n >= 512;
+  if (packed) return n >= 1024 || n * k >= 6 << 20;
+  return f32 ? n >= 1536 || n * k >= 9 << 20 : n >= 2048;
+}
+
 template <bool PACKED>
 int launch_quantize(const char* fn, const void* w, int w_dtype, int64_t n, int64_t k, int8_t* q, float* scale,
                     void* stream) {
@@ -318,7 +335,8 @@ int launch_quantize(const char* fn, const void* w, int w_dtype, int64_t n, int64
   // rows of whole, aligned 16-byte pieces that fit the tile kernel's registers
   // and LDS: up to 12288 columns
   const int vec = w_dtype == PGS_DTYPE_F32 ? 4 : 8;
-  if (k > 0 && k % vec == 0 && k <= kTileMaxK && aligned(w, 16) && aligned(q, PACKED ? 16 : vec)) {
+  if (k > 0 && k % vec == 0 && k <= kTileMaxK && aligned(w, 16) && aligned(q, PACKED ? 16 : vec) &&
+      tile_quantizer(PACKED, w_dtype == PGS_DTYPE_F32, n, k)) {
     const dim3 grid(static_cast<unsigned>(PACKED ? (n + 15) / 16 * 2 : (n + 7) / 8));
     const int kk = static_cast<int>(k), kbb = static_cast<int>(kb);
 #define PGS_QUANT_TILE(BF, NV)                                                                                   \

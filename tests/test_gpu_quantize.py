@@ -273,6 +273,17 @@ def test_tile_kernel_edges(gpu, n, k, dtype):
     np.testing.assert_array_equal(qw.scale.cpu().numpy(), s_ref)
 
 
+# both sides of each line between the one-row and the eight-row quantizer:
+# packed with padding (512 rows above 5120 columns), packed without (1024 rows
+# or 6 Mi weights), row-major fp32 (1536 rows or 9 Mi weights) and bf16 (2048)
+@pytest.mark.parametrize("n,k", [(511, 5128), (513, 5128), (1008, 1024), (1024, 64), (512, 12288), (496, 12288), (1535, 8),
+                                 (1537, 1032), (769, 12288), (2047, 2048), (2049, 2056), (2050, 4), (2063, 5120),
+                                 (2049, 1024), (2052, 2048), (2051, 12288)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_quantizer_row_counts(gpu, n, k, dtype):
+    test_tile_kernel_edges(gpu, n, k, dtype)
+
+
 @pytest.mark.parametrize("n,k", [(5, 3), (9, 4), (77, 5), (50, 7), (64, 8), (33, 9), (11, 12), (70, 1031), (16, 4104)])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
 def test_dequantize_pieces_across_rows(gpu, n, k, dtype):
