@@ -222,12 +222,14 @@ __global__ __launch_bounds__(kQuantThreads) void quantize_rows_kernel(
 // side: full lines both ways): the E weights of an item lie in one row or, for
 // k >= E, at most two.  IDX: 32-bit index arithmetic where the element count
 // allows (one division per item).  Quantizing and dequantizing a [16000, 8000]
-// fp32 weight row-major: 329 -> 244 us (5.2 TB/s).
-template <int OUT, typename IDX>
+// fp32 weight row-major: 329 -> 244 us (5.2 TB/s).  ITEMS: one for up to 4 Mi
+// weights, whose time is one thread's chain (bf16 of [976, 2048], with 1 / 2 / 4
+// items 2.80 / 2.91 / 3.47 us), else two ([31250, 2048] 33.9 / 30.9 / 31.2).
+template <int OUT, typename IDX, int ITEMS>
 __global__ __launch_bounds__(256) void dequantize_flat_kernel(const int8_t* __restrict__ q,
                                                               const float* __restrict__ scale, IDX n, IDX k,
                                                               IDX total, void* __restrict__ out) {
-  constexpr int E = OUT == PGS_DTYPE_F32 ? 4 : 8, ITEMS = 4;
+  constexpr int E = OUT == PGS_DTYPE_F32 ? 4 : 8;
   const IDX first = (static_cast<IDX>(blockIdx.x) * (256 * ITEMS) + threadIdx.x) * E;
   uint32_t wv[ITEMS][E / 4];
   float s0[ITEMS], s1[ITEMS];
@@ -282,15 +284,20 @@ __global__ __launch_bounds__(256) void dequantize1_kernel(const int8_t* __restri
 template <int OUT>
 int launch_dequant(const int8_t* q, const float* scale, int64_t n, int64_t k, void* out, hipStream_t st) {
   const int64_t total = n * k;
-  constexpr int E = OUT == PGS_DTYPE_F32 ? 4 : 8, PER = 256 * 4 * E;
-  if (k >= E && aligned(q, 8) && aligned(out, 16)) {
-    const unsigned blocks = static_cast<unsigned>((total + PER - 1) / PER);
-    if (total + PER < (1ll << 32))
-      hipLaunchKernelGGL((dequantize_flat_kernel<OUT, uint32_t>), dim3(blocks), dim3(256), 0, st, q, scale,
-                         static_cast<uint32_t>(n), static_cast<uint32_t>(k), static_cast<uint32_t>(total), out);
+  constexpr int E = OUT == PGS_DTYPE_F32 ? 4 : 8;
+  // (up to 512 Ki weights of rows of no whole 16: by element, without the second
+  // scale and the short last piece of the others: bf16 [97, 2047] 2.15 against 2.6 us)
+  if (k >= E && aligned(q, 8) && aligned(out, 16) && (k % 16 == 0 || total > (1 << 19))) {
+    const int64_t per = 256 * E * (total <= (4 << 20) ? 1 : 2);
+    const unsigned blocks = static_cast<unsigned>((total + per - 1) / per);
+    const dim3 grid(blocks), block(256);
+    const uint32_t n32 = static_cast<uint32_t>(n), k32 = static_cast<uint32_t>(k), t32 = static_cast<uint32_t>(total);
+    if (total <= (4 << 20))
+      hipLaunchKernelGGL((dequantize_flat_kernel<OUT, uint32_t, 1>), grid, block, 0, st, q, scale, n32, k32, t32, out);
+    else if (total + per < (1ll << 32))
+      hipLaunchKernelGGL((dequantize_flat_kernel<OUT, uint32_t, 2>), grid, block, 0, st, q, scale, n32, k32, t32, out);
     else
-      hipLaunchKernelGGL((dequantize_flat_kernel<OUT, int64_t>), dim3(blocks), dim3(256), 0, st, q, scale, n, k, total,
-                         out);
+      hipLaunchKernelGGL((dequantize_flat_kernel<OUT, int64_t, 2>), grid, block, 0, st, q, scale, n, k, total, out);
   } else {
     const int64_t blocks = (total + 255) / 256;
     hipLaunchKernelGGL(dequantize1_kernel<OUT>, dim3(static_cast<unsigned>(blocks)), dim3(256), 0, st, q, scale,

@@ -299,6 +299,13 @@ def test_dequantize_pieces_across_rows(gpu, n, k, dtype):
     assert torch.equal(qw.dense().cpu(), ref)
 
 
+# by element up to 512 Ki weights of odd rows, then one item per thread up to 4 Mi, then two
+@pytest.mark.parametrize("n,k", [(508, 1031), (509, 1031), (4069, 1031), (4068, 1031), (4, 16), (2048, 2048), (2049, 2048)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_dequantize_item_counts(gpu, n, k, dtype):
+    test_dequantize_pieces_across_rows(gpu, n, k, dtype)
+
+
 def test_dequantize_above_32_bit_indices(gpu):
     n, k = 65600, 65544
     q = torch.randint(-127, 128, (64, k), dtype=torch.int8, device=gpu).repeat(n // 64, 1)
