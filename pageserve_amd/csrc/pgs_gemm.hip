@@ -56,6 +56,7 @@ struct GemmArgs {
   int tiles;       // output tiles (tiles_m x weight-row tiles over all members)
   int splits;
   float* partials;
+  bool residuals;  // some member has one
 };
 
 // Split-K partial tile in lane order: [tile][split][mat][nt][mt][lane] x f32x4
@@ -1231,9 +1232,17 @@ __global__ __launch_bounds__(kThreads) void gemm_reduce_kernel(GemmArgs ga) {
   const int nb = n0 + wave * (BN / 4) + nt * 16 + 4 * (lane >> 4);
   if (m >= M) return;
   const Rows4<NMAT> e = rows4<NMAT>(a, g, N, nb);
-  const uint16_t* res = (NMAT == 2) ? nullptr : pick(a.res, g);
+  const uint16_t* res = nullptr;
   u32x2 rv = {0u, 0u};
-  if (NMAT == 1 && res) rv = residual4(res, vec_res(res, N), M, N, m, nb);
+  // (behind the partial loads, and on a flag that is the same for all: the pointer
+  // differs by lane.  On the pointer and in front of the partials it put its
+  // round trip before theirs also where there is no residual: down_proj [2048,
+  // 11008] at 33 / 64 tokens 12.7 / 14.1 against 12.3 / 13.6 us)
+  auto load_residual = [&] {
+    if (NMAT == 2 || !ga.residuals) return;
+    res = pick(a.res, g);
+    if (res) rv = residual4(res, vec_res(res, N), M, N, m, nb);
+  };
   const f32x4* part = reinterpret_cast<const f32x4*>(ga.partials) + static_cast<int64_t>(t) * ga.splits * NMAT * SLOTS;
   f32x4 v[NMAT];
   if constexpr (SPL > 0) {
@@ -1242,6 +1251,7 @@ __global__ __launch_bounds__(kThreads) void gemm_reduce_kernel(GemmArgs ga) {
     for (int mat = 0; mat < NMAT; ++mat)
 #pragma unroll
       for (int sp = 0; sp < SPL; ++sp) pv[mat][sp] = __builtin_nontemporal_load(part + (sp * NMAT + mat) * SLOTS + slot);
+    load_residual();
 #pragma unroll
     for (int mat = 0; mat < NMAT; ++mat) {
       v[mat] = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -1254,6 +1264,7 @@ __global__ __launch_bounds__(kThreads) void gemm_reduce_kernel(GemmArgs ga) {
       v[mat] = f32x4{0.f, 0.f, 0.f, 0.f};
       for (int sp = 0; sp < ga.splits; ++sp) v[mat] += part[(static_cast<int64_t>(sp) * NMAT + mat) * SLOTS + slot];
     }
+    load_residual();
   }
   void* y = (NMAT == 2) ? a.y[0] : pick(a.y, g);
   store_rows4<NMAT, OUT_F32>(N, m, nb, e, v[0], v[NMAT - 1], res != nullptr, rv, y, vec_out<OUT_F32>(y, N));
@@ -1781,6 +1792,7 @@ int launch_gemm(Problem& p, const GemmPlan& plan, hipStream_t st) {
   ga.tiles = plan.tiles;
   ga.splits = plan.splits;
   ga.partials = p.partials;
+  for (int i = 0; i < members; ++i) ga.residuals |= p.args.res[i] != nullptr;
   if (p.nmat == 2) return launch_plan<2, false>(p.x, ga, plan, st);
   return p.out_f32 ? launch_plan<1, true>(p.x, ga, plan, st) : launch_plan<1, false>(p.x, ga, plan, st);
 }
