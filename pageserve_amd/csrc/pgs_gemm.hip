@@ -1274,10 +1274,14 @@ template <int BM, int BN, int NMAT, bool OUT_F32>
 int launch_reduce(const GemmArgs& ga, hipStream_t st) {
   const int64_t slots = static_cast<int64_t>(ga.tiles) * BM * BN / 4;
   const dim3 grid(static_cast<unsigned>((slots + kThreads - 1) / kThreads));
+  // (three: six splits in pairs, which only the 128 x 128 tile has)
+  if constexpr (BM == 128 && BN == 128 && NMAT == 1)
+    if (ga.splits == 3) {
+      hipLaunchKernelGGL((gemm_reduce_kernel<BM, BN, NMAT, OUT_F32, 3>), grid, dim3(kThreads), 0, st, ga);
+      return check_launch("w8a16 gemm reduce kernel");
+    }
   if (ga.splits == 2)
     hipLaunchKernelGGL((gemm_reduce_kernel<BM, BN, NMAT, OUT_F32, 2>), grid, dim3(kThreads), 0, st, ga);
-  else if (ga.splits == 3)
-    hipLaunchKernelGGL((gemm_reduce_kernel<BM, BN, NMAT, OUT_F32, 3>), grid, dim3(kThreads), 0, st, ga);
   else if (ga.splits == 4)
     hipLaunchKernelGGL((gemm_reduce_kernel<BM, BN, NMAT, OUT_F32, 4>), grid, dim3(kThreads), 0, st, ga);
   else if (ga.splits == 8)
