@@ -268,9 +268,11 @@ int pgs_w8a16_swiglu(const void* x, const int8_t* qp_gate, const float* s_gate,
 /*
  * Replaces h = rms_norm(x, weight, eps) followed by the q/k/v projections of
  * h -- engine/model.py:166 (rms_norm at :29-34) and :168-170 -- with one
- * launch where the plan allows (m <= 32 tokens, K % 64 == 0 and at most 2048
- * above 4 tokens, no K split, bf16 outputs, 16-byte aligned norm weight): the
- * kernel normalises the activations it loads, with the reference's roundings
+ * launch where the plan allows (K % 64 == 0, no K split, bf16 outputs, 16-byte
+ * aligned norm weight, and m <= 4 tokens, or m <= 16 with K <= 2048 and few
+ * enough output rows that the workgroups repeating the norm cost less than its
+ * launch: at K <= 1024 16384 rows for m <= 8 and 8192 above, at longer K 4096 and
+ * none): the kernel normalises the activations it loads, with the reference's roundings
  * (h = bf16(weight * bf16(x * r)), r = 1/sqrt(mean(x^2) + eps) in fp32);
  * otherwise pgs_rmsnorm into the workspace, then pgs_w8a16_linear_group.
  * The fp32 sum of squares is formed in a fixed order (deterministic) that
@@ -285,8 +287,8 @@ int pgs_w8a16_rmsnorm_linear_group(const void* x, const void* norm_weight, float
 /*
  * Replaces h = rms_norm(x, weight, eps); silu(F.linear(h, Wg)) * F.linear(h,
  * Wu) -- engine/model.py:187-189 -- with one launch where the plan allows
- * (same conditions and roundings as pgs_w8a16_rmsnorm_linear_group),
- * otherwise pgs_rmsnorm into the workspace, then pgs_w8a16_swiglu.
+ * (m <= 4 tokens; the other conditions and the roundings of
+ * pgs_w8a16_rmsnorm_linear_group), otherwise pgs_rmsnorm into the workspace, then pgs_w8a16_swiglu.
  */
 int pgs_w8a16_rmsnorm_swiglu(const void* x, const void* norm_weight, float eps,
                              const int8_t* qp_gate, const float* s_gate,
@@ -300,9 +302,11 @@ int pgs_w8a16_rmsnorm_swiglu(const void* x, const void* norm_weight, float eps,
  * apply_rope(q), apply_rope(k) and v, with the reference's roundings (the bf16
  * projection, then pgs_rope's three).  cos / sin: bf16 [m, head_dim]; outs[0].n
  * and outs[1].n are whole heads of head_dim.  One launch at up to 32 tokens
- * where the norm runs inside the projection and head_dim % 32 == 0 (the two
- * halves of a head are then computed side by side); the separate kernels
- * otherwise.  Workspace: pgs_w8a16_rmsnorm_workspace_bytes of the three.
+ * where the norm runs inside the projection (above 4 tokens K <= 2048 and, since
+ * the rotation's launch is saved too, up to 16384 / 8192 output rows for m <= 8 / 16
+ * at K <= 1024, 8192 / 4096 at longer K, and 4096 for m <= 32) and head_dim % 32 == 0
+ * (the two halves of a head are then computed side by side); the separate
+ * kernels otherwise.  Workspace: pgs_w8a16_rmsnorm_workspace_bytes of the three.
  */
 int pgs_w8a16_rmsnorm_qkv_rope(const void* x, const void* norm_weight, float eps,
                                const pgs_linear_out* outs, const void* cos,

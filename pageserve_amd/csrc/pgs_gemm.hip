@@ -1570,7 +1570,10 @@ int launch_plan(const uint16_t* x, const GemmArgs& ga, const GemmPlan& plan, hip
 // and the partials' bytes, written and read (5 and 6.5 TB/s).  Measured in a
 // layer, GEMM + reduce us, kg = 1 -> 2: down_proj [2048, 11008] at 2048 tokens
 // (two splits) 104 -> 99, at 640 (eight -> six) 49 -> 42, at 512 (eight) 37 ->
-// 35; but at 1024 (four) 58 -> 60 and at 1450, 192 tiles, 12 us more.
+// 35; but at 1024 (four) 58 -> 60 and at 1450, 192 tiles, 12 us more.  Against
+// every split forced, and the unsplit pipelined tile where that is taken, over
+// 187 sizes (512 .. 4096 rows, 65 .. 172 steps, 300 .. 2048 tokens), the choice is
+// within 3 % of the best at 177 and within 10 % at all.
 struct LongSplit {
   int splits, kg;
   double cost;
@@ -1581,6 +1584,8 @@ static LongSplit long_k_split(int64_t tiles, int kb) {
   double best_cost = 0;
   for (int kg = 2; kg >= 1; --kg)
     for (int sp = 2; sp <= 8; sp += 2) {
+      // (six partial tiles per output have no unrolled reduce: by 3 .. 57 % behind
+      // the best other split at 179 of 187 sizes, at most 1 % ahead of it)
       if (kg == 1 && sp == 6) continue;
       const int64_t wgs = tiles * (sp / kg);
       const double rounds = kg == 2 ? 1.1 * static_cast<double>((wgs + 255) / 256)
@@ -1726,7 +1731,9 @@ GemmPlan plan_gemm(int m, int k, int nmat, const int32_t* n, int members, bool c
   // 14.8 / 20.7 / 23.7, [1152, 896] at 1501 11.0 -> 9.7; more tiles are slower
   // (560: 28.9 vs 30.0).  Long K of up to 96 steps: where its steps cost less
   // than the split above, in the same measure ([896, 4864] at 1280 / 1501 / 2048
-  // tokens 27.3 / 29.8 / 36.7 before either -> 22.8 / 23.4 / 25.7).
+  // tokens 27.3 / 29.8 / 36.7 before either -> 22.8 / 23.4 / 25.7); beyond, it wins
+  // at some sizes and loses at others ([2048, 7168] at 640 / 1024 tokens 28.9 / 39.5
+  // split, 30.6 / 36.5 unsplit; [2048, 11008] 36.7 / 52.4, 43.4 / 53.2).
   if (nmat == 1 && k % kBK == 0 && p.bn == kBN && m > 128) {
     const int64_t t64 = tiles_for(64);
     int kg = 0;

@@ -559,10 +559,11 @@ def linear_group(x: torch.Tensor, weights: list["QuantizedWeight"], biases: list
 def rmsnorm_linear_group(x: torch.Tensor, norm_weight: torch.Tensor, eps: float, weights: list["QuantizedWeight"],
                          biases: list | None = None, out_dtype: torch.dtype = torch.bfloat16) -> list[torch.Tensor]:
     """``h = rms_norm(x, norm_weight, eps)`` then the projections of ``h``
-    (engine/model.py:166-170), in one launch for up to 32 tokens (above 4 of
-    them for K up to 2048; the kernel normalises the activations it loads; its
-    fixed-order sum of squares may make ``h`` differ from :func:`rmsnorm` in
-    the last bf16 bit), otherwise :func:`rmsnorm` then :func:`linear_group`."""
+    (engine/model.py:166-170), in one launch for up to 4 tokens and, where few
+    enough workgroups repeat the norm (K up to 2048, q|k|v's widths), for up to
+    16 (the kernel normalises the activations it loads; its fixed-order sum of
+    squares may make ``h`` differ from :func:`rmsnorm` in the last bf16 bit),
+    otherwise :func:`rmsnorm` then :func:`linear_group`."""
     return _linear_group(x, weights, biases, out_dtype, norm_weight, eps)
 
 
@@ -589,8 +590,8 @@ def _linear_group(x, weights, biases, out_dtype, norm_weight, eps) -> list[torch
 
 def _rmsnorm_qkv_rope(x, norm_weight, eps, weights, biases, cos, sin, head_dim) -> list[torch.Tensor]:
     """:func:`rmsnorm_linear_group` of q, k and v, then :func:`rope_qk` of the
-    first two (engine/model.py:166-173), in one launch where the norm runs
-    inside the projection and the heads allow it.  ``q`` and ``k`` must be
+    first two (engine/model.py:166-173), in one launch for up to 32 tokens where
+    the norm runs inside the projection and the heads allow it.  ``q`` and ``k`` must be
     whole heads of ``head_dim``."""
     if not weights[0].qp.is_cuda:
         raise RuntimeError("W8A16 linear: the weight must be on a ROCm GPU (call .to('cuda') first)")
@@ -615,8 +616,8 @@ def swiglu(x: torch.Tensor, gate: "QuantizedWeight", up: "QuantizedWeight") -> t
 def rmsnorm_swiglu(x: torch.Tensor, norm_weight: torch.Tensor, eps: float, gate: "QuantizedWeight",
                    up: "QuantizedWeight") -> torch.Tensor:
     """``h = rms_norm(x, norm_weight, eps)`` then :func:`swiglu` of ``h``
-    (engine/model.py:187-189), in one launch for up to 32 tokens (as
-    :func:`rmsnorm_linear_group`)."""
+    (engine/model.py:187-189), in one launch for up to 4 tokens, otherwise
+    :func:`rmsnorm` then :func:`swiglu`."""
     return _swiglu(x, gate, up, norm_weight, eps)
 
 

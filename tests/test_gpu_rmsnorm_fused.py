@@ -1,8 +1,8 @@
 """rms_norm fused into the projections that consume it (engine/model.py:166-170
 and :187-189): ``rmsnorm_linear_group`` and ``rmsnorm_swiglu``.
 
-Up to four tokens (a group up to 32 of them where K fits the launch's
-registers), K % 64 == 0 and a bf16 output run one launch whose skinny kernel
+Up to four tokens (a group up to 32 of them where few enough workgroups repeat
+the norm), K % 64 == 0 and a bf16 output run one launch whose skinny kernel
 normalises the activations it loads; every other case runs the RMSNorm kernel
 into the workspace and then the plain projection.  Both are checked:
 
