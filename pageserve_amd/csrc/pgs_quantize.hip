@@ -310,13 +310,13 @@ int launch_dequant(const int8_t* q, const float* scale, int64_t n, int64_t k, vo
 // and wait for all of a row's loads, so it needs about one per CU; below that the
 // n workgroups of the one-row kernel, small and read from L2 the second time, end
 // sooner (one-row -> eight-row kernel, us).  Row-major fp32 [n, 2048] at n = 256 /
-// 1024 / 1536 / 4096: 3.0 -> 4.2, 4.4 -> 4.7, 5.3 -> 5.3, 10.9 -> 9.0, and [n, 8192]
-// at 256 / 1024 / 1536: 6.7 -> 10.7, 12.3 -> 12.8, 18.4 -> 15.4; bf16 [n, 2048] at
+// 1024 / 1536 / 4096: 3.0 -> 4.2, 4.4 -> 4.7, 5.3 -> 5.3, 10.9 -> 9.0, and [n, 12288]
+// at 256 / 512 / 1024: 9.0 -> 12.3, 12.9 -> 13.5, 18.7 -> 16.1; bf16 [n, 2048] at
 // 1024 / 2048 / 4096: 3.8 -> 4.2, 5.0 -> 5.1, 7.6 -> 7.1.  Packed, whose one-row kernel
 // writes parts of lines: fp32 [n, 2048] at 256 / 1024: 3.4 -> 4.4, 5.4 -> 4.9, [n,
 // 12288] at 256 / 512: 10.7 -> 12.8, 16.6 -> 14.1.  Where padding is to be cleared the
 // one-row kernel needs a fill launch: [150, 2048] 4.7 -> 4.1, only longer rows are
-// sooner done with it ([300 | 600, 8192] 10.2 -> 11.0, 13.9 -> 11.8).
+// sooner done with it ([150 | 600, 12288] 11.6 -> 12.4, 21.6 -> 14.6).
 bool tile_quantizer(bool packed, bool f32, int64_t n, int64_t k) {
   if (packed && (n % 16 != 0 || k % 64 != 0)) return k <= 5120 || n >= 512;
   if (packed) return n >= 1024 || n * k >= 6 << 20;
@@ -340,7 +340,9 @@ int launch_quantize(const char* fn, const void* w, int w_dtype, int64_t n, int64
   if (int rc = require_device(fn, st)) return rc;
   const int64_t kb = packed_kblocks(k);
   // rows of whole, aligned 16-byte pieces that fit the tile kernel's registers
-  // and LDS: up to 12288 columns
+  // and LDS: up to 12288 columns, in steps whose unused loads are few (the step at
+  // 8192: fp32 [11008, 5128] row-major / packed 59.0 / 66.8 us, 74.3 / 76.8 in the
+  // loads of 12288; 65.6 KB of LDS leave room for a second packed workgroup)
   const int vec = w_dtype == PGS_DTYPE_F32 ? 4 : 8;
   if (k > 0 && k % vec == 0 && k <= kTileMaxK && aligned(w, 16) && aligned(q, PACKED ? 16 : vec) &&
       tile_quantizer(PACKED, w_dtype == PGS_DTYPE_F32, n, k)) {
@@ -352,11 +354,13 @@ int launch_quantize(const char* fn, const void* w, int w_dtype, int64_t n, int64
       if (k <= 1024) PGS_QUANT_TILE(false, 2);
       else if (k <= 2048) PGS_QUANT_TILE(false, 4);
       else if (k <= 5120) PGS_QUANT_TILE(false, 10);
+      else if (k <= 8192) PGS_QUANT_TILE(false, 16);
       else PGS_QUANT_TILE(false, 24);
     } else {
       if (k <= 1024) PGS_QUANT_TILE(true, 1);
       else if (k <= 2048) PGS_QUANT_TILE(true, 2);
       else if (k <= 5120) PGS_QUANT_TILE(true, 5);
+      else if (k <= 8192) PGS_QUANT_TILE(true, 8);
       else PGS_QUANT_TILE(true, 12);
     }
 #undef PGS_QUANT_TILE

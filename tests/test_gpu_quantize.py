@@ -278,7 +278,7 @@ def test_tile_kernel_edges(gpu, n, k, dtype):
 # or 6 Mi weights), row-major fp32 (1536 rows or 9 Mi weights) and bf16 (2048)
 @pytest.mark.parametrize("n,k", [(511, 5128), (513, 5128), (1008, 1024), (1024, 64), (512, 12288), (496, 12288), (1535, 8),
                                  (1537, 1032), (769, 12288), (2047, 2048), (2049, 2056), (2050, 4), (2063, 5120),
-                                 (2049, 1024), (2052, 2048), (2051, 12288)])
+                                 (2049, 1024), (2052, 2048), (2051, 12288), (2049, 8192), (2049, 8200)])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 def test_quantizer_row_counts(gpu, n, k, dtype):
     test_tile_kernel_edges(gpu, n, k, dtype)
