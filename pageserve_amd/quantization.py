@@ -593,6 +593,9 @@ def _rmsnorm_qkv_rope(x, norm_weight, eps, weights, biases, cos, sin, head_dim) 
     first two (engine/model.py:166-173), in one launch for up to 32 tokens where
     the norm runs inside the projection and the heads allow it.  ``q`` and ``k`` must be
     whole heads of ``head_dim``."""
+    biases = list(biases) if biases is not None else [None] * len(weights)
+    if len(biases) != len(weights):
+        raise ValueError("one bias (or None) per weight")
     if not weights[0].qp.is_cuda:
         raise RuntimeError("W8A16 linear: the weight must be on a ROCm GPU (call .to('cuda') first)")
     ops = [w._launch_operands() for w in weights]
@@ -603,8 +606,7 @@ def _rmsnorm_qkv_rope(x, norm_weight, eps, weights, biases, cos, sin, head_dim) 
     c, s = _rope_tables(cos, sin, m, head_dim, dev)
     qs, ss, ns = [o[0] for o in ops], [o[1] for o in ops], tuple(o[2] for o in ops)
     ws, ws_bytes, _buf = _ws_args(dev, x, k, ns, False, True)
-    return _native.load_host().qkv_rope(x, qs, ss, list(biases) if biases is not None else [None] * 3, ns, k,
-                                        norm_weight, eps, c, s, head_dim, ws, ws_bytes)
+    return _native.load_host().qkv_rope(x, qs, ss, biases, ns, k, norm_weight, eps, c, s, head_dim, ws, ws_bytes)
 
 
 def swiglu(x: torch.Tensor, gate: "QuantizedWeight", up: "QuantizedWeight") -> torch.Tensor:

@@ -107,6 +107,11 @@ def test_decode_chain_takes_empty_biases_as_none(monkeypatch, none):
     assert _chain_tail(monkeypatch, True, none) == [None, None, None]
 
 
+def test_decode_chain_wants_a_bias_or_none_per_weight(monkeypatch):
+    with pytest.raises(ValueError, match="one bias"):
+        _chain_tail(monkeypatch, True, [None, None])
+
+
 def test_decode_chain_says_where_its_weights_belong(monkeypatch):
     with pytest.raises(RuntimeError, match=r"ROCm GPU \(call .to\('cuda'\) first\)"):
         _chain_tail(monkeypatch, False, None)
